@@ -29,6 +29,16 @@ struct GridItem {       // one gridding work item: part of one tile's visit list
   int slot;             // -1: write the tile to the grid; else partial slot
   int pad0, pad1, pad2;
 };
+// 2D matrix-core scatter: what one wave does -- its part [vbeg, vend) of an
+// item's visit list, which g waves of the block (wave - sub .. wave - sub + g - 1)
+// share.  frame -1: nothing.
+struct GmWave {
+  int frame, tile, vbeg, vend, slot, g, sub, pad;
+};
+struct GmShape {       // launch shape of the 2D matrix-core scatter at C coils
+  int waves, groups;   // waves per block, coil groups
+};
+GmShape gm_shape(int C);
 struct ReduceItem {     // sums the partial slots of one heavy tile
   int frame, tile, slot0, nslots;
 };
@@ -269,6 +279,7 @@ struct GridArgs {
   float2* grid;
   float2* partial;
   const GridItem* items;
+  const GmWave* gwaves; // matrix-core kernel (2D): gm_shape(C).waves entries per block
   const int* visits;
   const int* fdone;
   int d, taps, C, T, CGW, rowstride;
@@ -344,7 +355,7 @@ struct Plan {
                                       // 3D 1: (sample, plane), 2: (sample, plane, parity)
   bool use_grid_batched = true;       // batched visit lists (else one visit at a time)
   bool use_grid_reg = true;           // 2D: register accumulation, lane = cell of an 8x8 tile
-  bool use_grid_mfma = false;         // 2D: scatter on the matrix cores (k_grid_mfma)
+  bool use_grid_mfma = false;         // scatter on the matrix cores (k_grid_mfma, k_grid_mfma3)
   int grid_cgr = 16;                  // coils per wave in the register kernel
   bool use_grid_atomic = false;       // LDS float atomics variant (kept for comparison)
   bool use_grid_sweep = false;        // 2D: line-sweep scatter (kernels_sweep.hip) where supported
@@ -384,6 +395,8 @@ struct Plan {
   int n_tile_items = 0;
   GridItem* grid_items = nullptr;
   int n_grid_items = 0;
+  GmWave* gm_waves = nullptr;         // 2D matrix-core scatter: gm_shape(C).waves entries per block
+  int n_gm_blocks = 0;
   ReduceItem* reduce_items = nullptr;
   int n_reduce_items = 0;
   int* visits = nullptr;
@@ -537,7 +550,7 @@ void launch_interp_lds(const SampArgs& a, const int4* items, int nitems, int T, 
 size_t grid_batched_lds(int d, int T, int taps, int CG, int rowstride);
 void launch_grid_atomic(const GridArgs& a, const int4* vrec, int cg, int nitems, int ncgroups, hipStream_t s);
 void launch_grid_reg(const GridArgs& a, const int4* vrec, int cgr, int nitems, int ncgroups, hipStream_t s);
-void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s);
+void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nblocks, hipStream_t s);
 void launch_grid_mfma3(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s);
 int sweep_groups(int C);
 bool grid_sweep_supported(int taps, int C);

@@ -20,6 +20,7 @@
 namespace cgs {
 
 typedef float gf32x16 __attribute__((ext_vector_type(16)));   // MFMA 32x32 accumulator
+typedef float gf32x4 __attribute__((ext_vector_type(4)));     // MFMA 16x16 accumulator
 
 // v + (v of the lane that the DPP control CTRL selects); lanes whose source
 // lies outside the 16-lane row add zero
@@ -1055,165 +1056,271 @@ void launch_grid_reg(const GridArgs& a, const int4* vrec, int cgr, int nitems, i
 
 // ---------------------------------------------------------------------------
 // adjoint B^T on the matrix cores (2D, 8x8 tiles).  The tile's grid values are
-// D[cell][col] (64 cells x the real columns re/im of CC = 16 NT coils) and the
-// work item's visit list is a K dimension: D += W[cell][visit] Y[visit][col],
-// with W the visit's separable window weight at the cell (0 outside its
-// footprint) and Y its weighted data.  One wave per work item; every
-// v_mfma_f32_32x32x2f32 (FP32 products and sums) takes two visits for one
-// (32-cell half, 32-column tile).  The zero weights of cells outside a visit's
-// footprint cost matrix-core cycles instead of VALU issue, and the weights are
-// formed while the previous products run.  Operand layout: A lane l =
-// W[l % 32][l / 32], B lane l = Y[l / 32][l % 32], accumulator register r of
-// lane l = D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].  Each cell still has one
-// owner and visits are applied in list order: deterministic, no atomics.
-
-template <int NT, int TAPS, int B>
-__global__ void __launch_bounds__(256) k_grid_mfma(GridArgs a, const int4* __restrict__ vrec, int nitems) {
-  constexpr int NPSI = 2 * TAPS, NCOL = 32 * NT, CC = 16 * NT;
-  constexpr int WAVE_FLOATS = B * NCOL + B * NPSI + B * 4;
-  extern __shared__ float shf[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int item = blockIdx.x * 4 + wave;
-  if (item >= nitems) return;          // waves of a block never synchronise with each other
-  const GridItem it = a.items[item];
-  if (a.fdone && a.fdone[it.frame]) return;
-  float* wy = shf + wave * WAVE_FLOATS;           // [B][NCOL]
-  float* wpsi = wy + B * NCOL;                    // [B][NPSI]
-  int4* wrec = (int4*)(wpsi + B * NPSI);          // [B]
-  const int cbase = blockIdx.y * CC;
-  const int t0 = it.tile % a.nt0, t1 = it.tile / a.nt0;
-  const int ts0 = t0 * 8, ts1 = t1 * 8;
-  const int te0 = min(8, a.n0 - ts0), te1 = min(8, a.n1 - ts1);
-  const int i = lane & 31, kk = lane >> 5;
-  const int cx = i & 7, cy0 = i >> 3, cy1 = 4 + (i >> 3);   // A rows: cells i and 32 + i
-  gf32x16 acc[2][NT];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[h][t][r] = 0.f;
-
-  for (int vb = it.vbeg; vb < it.vend; vb += B) {
-    const int nb = min(B, it.vend - vb);
-    // visits past nb (the odd one of the last pair) get a footprint outside
-    // every tile and zero data, so the pair loop below needs no branch
-    if (lane < B) wrec[lane] = (lane < nb) ? vrec[vb + lane] : make_int4(0, 0x40004000, 0, 0);
-    __builtin_amdgcn_wave_barrier();
-    {
-      // every load of the batch in flight before the first LDS write
-      constexpr int UP = (B * NPSI + 63) / 64, UY = (B * CC + 63) / 64;
-      float pv[UP];
-      float2 yv[UY];
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int idx = lane + 64 * u;
-        pv[u] = 0.f;
-        if (idx < nb * NPSI) {
-          const int v = idx / NPSI, q = idx - v * NPSI;
-          pv[u] = a.psi[(int64_t)wrec[v].x * NPSI + q];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UY; ++u) {   // float2 units: (visit, coil)
-        const int idx = lane + 64 * u;
-        yv[u] = make_float2(0.f, 0.f);
-        if (idx < nb * CC) {
-          const int v = idx / CC, c = idx - v * CC;
-          if (cbase + c < a.C) {
-            const int smp = wrec[v].x;
-            yv[u] = a.y[(int64_t)smp * a.C + cbase + c];
-            if (a.w) { const float ww = a.w[smp]; yv[u].x *= ww; yv[u].y *= ww; }
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int idx = lane + 64 * u;
-        if (idx < nb * NPSI) wpsi[idx] = pv[u];
-      }
-#pragma unroll
-      for (int u = 0; u < UY; ++u) {
-        const int idx = lane + 64 * u;
-        if (idx < B * CC) ((float2*)wy)[idx] = yv[u];   // zeros past nb
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    // branch-free: the four LDS reads of a pair depend only on its record, and
-    // out-of-footprint weights are selected to zero (reads stay in the batch)
-    for (int v = 0; v < nb; v += 2) {
-      const int vk = v + kk;   // this lane's visit of the pair (K index); vk <= nb < B or vk < B
-      const int4 rc = wrec[vk];
-      const int rel0 = (int)(short)(rc.y & 0xffff), rel1 = (int)(short)(rc.y >> 16);
-      const float* ps = wpsi + vk * NPSI;
-      const int dx = cx - rel0, dy0 = cy0 - rel1, dy1 = cy1 - rel1;
-      const bool okx = (unsigned)dx < (unsigned)TAPS;
-      const bool ok0 = okx && (unsigned)dy0 < (unsigned)TAPS, ok1 = okx && (unsigned)dy1 < (unsigned)TAPS;
-      const float px = ps[okx ? dx : 0];
-      const float q0 = ps[TAPS + (ok0 ? dy0 : 0)], q1 = ps[TAPS + (ok1 ? dy1 : 0)];
-      float bv[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) bv[t] = wy[vk * NCOL + 32 * t + i];
-      const float w0 = ok0 ? px * q0 : 0.f, w1 = ok1 ? px * q1 : 0.f;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(w0, bv[t], acc[0][t], 0, 0, 0);
-        acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(w1, bv[t], acc[1][t], 0, 0, 0);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-
-  const int ncol = 2 * min(CC, a.C - cbase);   // real columns of this coil group
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int cell = 32 * h + 8 * (r >> 2) + 4 * kk + (r & 3);
-      const int x0 = cell & 7, x1 = cell >> 3;
-      if (x0 >= te0 || x1 >= te1) continue;
-      float* out;
-      if (it.slot < 0) {
-        const int64_t l = (ts0 + x0) + (int64_t)a.n0 * (ts1 + x1);
-        out = (float*)(a.grid + ((int64_t)it.frame * a.ntot + l) * a.C + cbase);
-      } else {
-        out = (float*)(a.partial + ((int64_t)it.slot * a.tilecells + x0 + 8 * x1) * a.C + cbase);
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int col = 32 * t + i;
-        if (col < ncol) out[col] = acc[h][t][r];
-      }
-    }
+// D[cell][col] (64 cells x the real columns re/im of a coil group) and the work
+// item's visit list is a K dimension: D += W[cell][visit] Y[visit][col], with W
+// the visit's separable window weight at the cell (0 outside its footprint) and
+// Y its weighted data.  R = 32 (16 coils): v_mfma_f32_32x32x2f32, two visits
+// for one 32-cell half; R = 16 (8 coils): v_mfma_f32_16x16x4f32, four visits for
+// one 16-cell quarter.  FP32 products and sums.  Operand layout: A lane l =
+// W[l % R][l / R], B lane l = Y[l / R][l % R], accumulator register r of lane l
+// = D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32] (R = 32), D[4 (l / 16) + r][l % 16]
+// (R = 16).
+//
+// What bounds it: the matrix-core work is 28-38 us at 256^2 x 32 coils, but each
+// visit must be brought and placed first.  A batch of 16 visits is staged per
+// wave in LDS with the window values already on the tile's 8 + 8 axis cells
+// (density weight in the axis-0 factor), so a product's weight is one
+// multiplication of two LDS reads at immediate offsets (a version that placed
+// each visit's footprint per product had 25 vector instructions a product in a
+// chain of two LDS reads); the next batch's loads and the records of the one
+// after are in flight meanwhile, branch-free.  Lists are sorted by the axis-1
+// offset and products of a group no visit of eight meets are left out (27 % of
+// them).  Batches of 16, not 32: 94 instead of 114 registers, 5 waves a SIMD
+// (64 frames of 192^2 x 16 coils: 395 against 428 us).  Lists longer than a
+// wave's share are split: g = 1, 2, 4 or 8 waves of a block take contiguous
+// parts of one item's list and add their accumulators through LDS in wave order,
+// so the walk of the longest list (the k-space centre), one wave's serial chain,
+// does not set the launch's time.  Measured, one wave per item with per-product
+// placement -> this: 64^2 x 1 coil 63 -> 12 us, 128^2 x 8 coils 97 -> 15 us,
+// 216 x 162 x 12 coils 106 -> 34 us, 256^2 x 32 coils (205 824 samples) 154 ->
+// 81 us, 64 frames of 192^2 x 16 coils 650 -> 395 us.  Each cell has one owner
+// and a fixed order of sums: deterministic, no atomics.
+constexpr int kGmBatch = 16;   // visits staged at a time
+// LDS of a wave in floats: weights on the tile's axis cells, data, records,
+// density weights; at least one reduction round (16 registers)
+constexpr int gm_wave_floats(int cols) {
+  return kGmBatch * (16 + cols + 3) > 1024 ? kGmBatch * (16 + cols + 3) : 1024;
 }
 
-template <int NT, int B>
-static void grid_mfma_taps(const GridArgs& a, const int4* vrec, int nitems, dim3 g, size_t shm, hipStream_t s) {
+// LDS written by some lanes of a wave and read by others: the wave's LDS
+// operations run in order, so only the compiler has to keep them so
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// R x R products (R / 2 coils a wave), NW waves a block; WIDE: C is even, so two
+// coils of a sample are one aligned 16-byte load
+template <int TAPS, int R, int NW, bool WIDE>
+__global__ void __launch_bounds__(64 * NW, 4) k_grid_mfma(GridArgs a, const int4* __restrict__ vrec, int ngroups) {
+  constexpr int B = kGmBatch, CC = R / 2, NPSI = 2 * TAPS;
+  constexpr int KV = 64 / R;                     // visits per product
+  constexpr int NH = 64 / R;                     // cell groups of R cells
+  constexpr int NR = R == 32 ? 16 : 4;           // accumulator registers per group
+  constexpr int WF = gm_wave_floats(R);
+  constexpr int UW = B * 16 / 64, UY = B * CC / 128;
+  __shared__ __attribute__((aligned(16))) float shf[NW * WF];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = blockIdx.x / ngroups;          // every coil group of a block's items together: the longest first
+  const GmWave it = a.gwaves[blk * NW + wave];
+  const bool active = it.frame >= 0 && !(a.fdone && a.fdone[it.frame]);
+  const int g = it.g, sub = it.sub;
+  if (g == 1 && !active) return;                 // waves of a shared item meet at barriers
+  float* wW = shf + wave * WF;                   // [B][16]: axis 0, axis 1 weights on the tile's cells
+  float* wY = wW + B * 16;                       // [B][R]
+  int2* wrec = (int2*)(wY + B * R);           // [B]: sample, packed tile offsets
+  float* wden = (float*)(wrec + B);              // [B]: density weight
+  const int cbase = (blockIdx.x - blk * ngroups) * CC;
+  const int ts0 = (it.tile % a.nt0) * 8, ts1 = (it.tile / a.nt0) * 8;
+  const int te0 = min(8, a.n0 - ts0), te1 = min(8, a.n1 - ts1);
+  const int i = lane % R, kk = lane / R;
+  gf32x16 acc32[R == 32 ? NH : 1];
+  gf32x4 acc16[R == 16 ? NH : 1];
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if constexpr (R == 32) acc32[h][r] = 0.f;
+      else acc16[h][r] = 0.f;
+    }
+
+  // Loads are branch-free (addresses clamped to valid ones, what they bring
+  // past the list or the footprint is dropped when it is staged): where two
+  // control paths merge the compiler would wait for every load in flight.
+  const int v0 = it.vbeg, v1 = active ? it.vend : it.vbeg;
+  const int axis = (lane >> 3) & 1, cell = lane & 7;
+  const float* dens = a.w ? a.w : a.psi;
+  float pv[UW], den = 0.f;
+  float4 yv[UY];
+  int4 rc = make_int4(0, 0, 0, 0);
+  unsigned in_foot = 0, need_next[NH], need[NH];
+  auto load_rec = [&](int vb) { rc = vrec[min(vb + (lane & (B - 1)), v1 - 1)]; };
+  auto put_rec = [&](int nb) {                   // past the list: a footprint outside every tile
+    const int ry = (lane & (B - 1)) < nb ? rc.y : 0x40004000;
+    if (lane < B) wrec[lane] = make_int2(rc.x, ry);
+    // visits whose footprint meets the axis-1 cells of group h (lists are sorted
+    // by their axis-1 offset, so runs of visits leave whole groups out)
+    const int r1 = ry >> 16;
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+      need_next[h] = (unsigned)__ballot(r1 < (h + 1) * (R / 8) && r1 + TAPS > h * (R / 8));
+    wave_lds_order();
+  };
+  auto load_batch = [&]() {
+    den = dens[rc.x];
+    in_foot = 0;
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+      const int2 r = wrec[u * 4 + (lane >> 4)];
+      const int t = cell - (axis ? (r.y >> 16) : (int)(short)(r.y & 0xffff));
+      in_foot |= (unsigned)((unsigned)t < (unsigned)TAPS) << u;
+      pv[u] = a.psi[(int64_t)r.x * NPSI + axis * TAPS + min(max(t, 0), TAPS - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < UY; ++u) {
+      const int idx = lane + 64 * u, v = idx / (CC / 2), c = cbase + 2 * (idx % (CC / 2));
+      const float2* src = a.y + (int64_t)wrec[v].x * a.C;   // columns past C are not stored
+      if constexpr (WIDE) {
+        yv[u] = *reinterpret_cast<const float4*>(src + min(c, a.C - 2));
+      } else {
+        const float2 p = src[min(c, a.C - 1)], q = src[min(c + 1, a.C - 1)];
+        yv[u] = make_float4(p.x, p.y, q.x, q.y);
+      }
+    }
+  };
+  auto put_batch = [&](int nb) {
+    if (lane < B) wden[lane] = a.w ? den : 1.f;
+    wave_lds_order();
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+      const float d = wden[u * 4 + (lane >> 4)];
+      wW[lane + 64 * u] = (in_foot >> u) & 1u ? pv[u] * (axis ? 1.f : d) : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < UY; ++u) {
+      const bool ok = (lane + 64 * u) / (CC / 2) < nb;
+      ((float4*)wY)[lane + 64 * u] = make_float4(ok ? yv[u].x : 0.f, ok ? yv[u].y : 0.f, ok ? yv[u].z : 0.f,
+                                                 ok ? yv[u].w : 0.f);
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h) need[h] = need_next[h];
+    wave_lds_order();
+  };
+  // weights of the lane's cell i of every group: axis-0 cell i & 7, axis-1 cell
+  // h R / 8 + (i >> 3); visits p0 .. p0 + 7
+  const float* px = wW + kk * 16 + (i & 7);
+  const float* qy = wW + kk * 16 + 8 + (i >> 3);
+  const float* by = wY + kk * R + i;
+  auto multiply8 = [&](int p0) {
+    float x[8 / KV], b[8 / KV];
+#pragma unroll
+    for (int u = 0; u < 8 / KV; ++u) {
+      x[u] = px[(p0 + u * KV) * 16];
+      b[u] = by[(p0 + u * KV) * R];
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      if (!((need[h] >> p0) & 0xffu)) continue;
+#pragma unroll
+      for (int u = 0; u < 8 / KV; ++u) {
+        const float w = x[u] * qy[(p0 + u * KV) * 16 + h * (R / 8)];
+        if constexpr (R == 32) acc32[h] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, b[u], acc32[h], 0, 0, 0);
+        else acc16[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, b[u], acc16[h], 0, 0, 0);
+      }
+    }
+  };
+  if (v0 < v1) {
+    load_rec(v0);
+    put_rec(v1 - v0);
+    load_batch();
+    load_rec(v0 + B);
+    int vb = v0;
+    for (; vb + B < v1; vb += B) {
+      put_batch(B);
+      put_rec(v1 - vb - B);
+      load_batch();
+      load_rec(vb + 2 * B);
+#pragma unroll
+      for (int p0 = 0; p0 < B; p0 += 8) multiply8(p0);
+      wave_lds_order();
+    }
+    put_batch(v1 - vb);
+    for (int p0 = 0; p0 < v1 - vb; p0 += 8) multiply8(p0);   // visits past the list are staged as zeros
+    wave_lds_order();
+  }
+
+  // four registers (quad q of group h) are four axis-0 neighbours x0 = xb ..
+  // xb + 3 of axis-1 cell x1: 4 h + q (R = 32), 2 h + (kk >> 1) (R = 16)
+  const int ncol = 2 * min(CC, a.C - cbase);
+  constexpr int NQ = NR / 4;                     // quads per group
+  auto store4 = [&](int k, float4 v) {
+    const int h = k / NQ, q = k % NQ;
+    const int x1 = R == 32 ? 4 * h + q : 2 * h + (kk >> 1);
+    const int xb = R == 32 ? 4 * kk : 4 * (kk & 1);
+    if (x1 >= te1 || i >= ncol) return;
+    const int64_t l = it.slot < 0 ? (int64_t)it.frame * a.ntot + ts0 + xb + (int64_t)a.n0 * (ts1 + x1)
+                                  : (int64_t)it.slot * a.tilecells + xb + 8 * x1;
+    float* out = (float*)((it.slot < 0 ? a.grid : a.partial) + l * a.C + cbase) + i;
+    const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (xb + j < te0) out[(int64_t)j * 2 * a.C] = e[j];
+  };
+  auto quad = [&](int k) {
+    const int h = k / NQ, q = k % NQ;
+    if constexpr (R == 32)
+      return make_float4(acc32[h][4 * q], acc32[h][4 * q + 1], acc32[h][4 * q + 2], acc32[h][4 * q + 3]);
+    else
+      return make_float4(acc16[h][0], acc16[h][1], acc16[h][2], acc16[h][3]);
+  };
+  if (g == 1) {
+#pragma unroll
+    for (int k = 0; k < NH * NQ; ++k) store4(k, quad(k));
+    return;
+  }
+  // shared item: rounds of four quads (16 registers, 4 KB a wave); quad k of a
+  // round is summed over the item's waves, in wave order, by wave k (mod g)
+#pragma unroll
+  for (int rd = 0; rd < NH * NQ / 4; ++rd) {
+    if (rd > 0) lds_barrier();                   // the round before is read
+    float4* mine = (float4*)wW;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mine[k * 64 + lane] = quad(4 * rd + k);
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if ((k & (g - 1)) != sub || !active) continue;
+      float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int j = 0; j < g; ++j) {
+        const float4 v = ((const float4*)(shf + (wave - sub + j) * WF))[k * 64 + lane];
+        t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+      }
+      store4(4 * rd + k, t);
+    }
+  }
+}
+
+// At most 8 coils: 16 x 16 products (half the matrix work of 32 x 32 ones whose
+// other columns are empty) and 8 waves a block, because such plans are small and
+// the walk of their longest list is what a launch waits for (64^2, 48 x 128
+// samples, 1 coil: 12 us, with 4 waves 16 us).  More coils: 4 waves, a smaller
+// unit of residency (256^2 x 32 coils: 81 us, with 8 waves 87 us).
+GmShape gm_shape(int C) { return C <= 8 ? GmShape{8, 1} : GmShape{4, (C + 15) / 16}; }
+
+template <int R, int NW>
+static void grid_mfma_taps(const GridArgs& a, const int4* vrec, int nblocks, int ng, hipStream_t s) {
+  const dim3 g((unsigned)nblocks * (unsigned)ng), b(64 * NW);
+#define CGS_GM(TP)                                                                                   \
+  do {                                                                                               \
+    if (a.C % 2 == 0) hipLaunchKernelGGL((k_grid_mfma<TP, R, NW, true>), g, b, 0, s, a, vrec, ng);    \
+    else hipLaunchKernelGGL((k_grid_mfma<TP, R, NW, false>), g, b, 0, s, a, vrec, ng);                \
+  } while (0)
   switch (a.taps) {
-    case 4: hipLaunchKernelGGL((k_grid_mfma<NT, 4, B>), g, dim3(256), shm, s, a, vrec, nitems); break;
-    case 6: hipLaunchKernelGGL((k_grid_mfma<NT, 6, B>), g, dim3(256), shm, s, a, vrec, nitems); break;
-    case 8: hipLaunchKernelGGL((k_grid_mfma<NT, 8, B>), g, dim3(256), shm, s, a, vrec, nitems); break;
-    case 10: hipLaunchKernelGGL((k_grid_mfma<NT, 10, B>), g, dim3(256), shm, s, a, vrec, nitems); break;
+    case 4: CGS_GM(4); break;
+    case 6: CGS_GM(6); break;
+    case 8: CGS_GM(8); break;
+    case 10: CGS_GM(10); break;
     default: break;
   }
+#undef CGS_GM
 }
 
-// NT column tiles of 16 coils per wave (CGS_GRID_MFMA_NT, default 1: more
-// waves per SIMD), visit batches of B (CGS_GRID_MFMA_B, 16 or 32)
-void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s) {
-  if (nitems == 0) return;
-  static const int nt_env = [] { const char* e = std::getenv("CGS_GRID_MFMA_NT"); return e ? std::atoi(e) : 1; }();
-  static const int b_env = [] { const char* e = std::getenv("CGS_GRID_MFMA_B"); return e ? std::atoi(e) : 32; }();
-  const int NT = (a.C <= 16 || nt_env != 2) ? 1 : 2;
-  const int B = b_env == 16 ? 16 : 32;
-  const int CC = 16 * NT;
-  const dim3 g((unsigned)((nitems + 3) / 4), (unsigned)((a.C + CC - 1) / CC));
-  const int npsi = 2 * a.taps;
-  const size_t shm = sizeof(float) * 4 * (B * 32 * NT + B * npsi + B * 4);
-  if (NT == 1 && B == 16) grid_mfma_taps<1, 16>(a, vrec, nitems, g, shm, s);
-  else if (NT == 1) grid_mfma_taps<1, 32>(a, vrec, nitems, g, shm, s);
-  else if (B == 16) grid_mfma_taps<2, 16>(a, vrec, nitems, g, shm, s);
-  else grid_mfma_taps<2, 32>(a, vrec, nitems, g, shm, s);
+void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nblocks, hipStream_t s) {
+  if (nblocks == 0) return;
+  const GmShape sh = gm_shape(a.C);
+  if (sh.waves == 8) grid_mfma_taps<16, 8>(a, vrec, nblocks, sh.groups, s);
+  else grid_mfma_taps<32, 4>(a, vrec, nblocks, sh.groups, s);
 }
 
 size_t grid_atomic_lds(int d, int T, int taps, int CG, int rowstride) {

@@ -433,7 +433,7 @@ static int gridding(Plan& p, const float2* y, bool weighted, const int* fl) {
   GridArgs a{};
   a.base = p.base; a.psi = p.psi; a.w = weighted ? p.w : nullptr;
   a.y = y; a.grid = p.grid; a.partial = p.partial;
-  a.items = p.grid_items; a.visits = p.visits; a.fdone = fl;
+  a.items = p.grid_items; a.gwaves = p.gm_waves; a.visits = p.visits; a.fdone = fl;
   a.d = p.d; a.taps = p.taps; a.C = p.C; a.T = p.T;
   const bool batched = p.use_grid_batched;
   a.CGW = batched ? p.grid_cg : p.grid_cg * p.grid_w;
@@ -467,7 +467,7 @@ static int gridding(Plan& p, const float2* y, bool weighted, const int* fl) {
     return CGS_OK;
   }
   if (p.d == 2 && p.T == 8 && p.use_grid_mfma) {
-    launch_grid_mfma(a, p.vrec, p.n_grid_items, p.stream);
+    launch_grid_mfma(a, p.vrec, p.n_gm_blocks, p.stream);
   } else if (p.d == 2 && p.T == 8 && p.use_grid_reg) {
     const int cgr = p.grid_cgr;
     launch_grid_reg(a, p.vrec, cgr, p.n_grid_items, (p.C + cgr - 1) / cgr, p.stream);
@@ -609,7 +609,8 @@ static void free_bins(Plan& p) {
 static void free_samples(Plan& p, bool sweep = true) {
   if (sweep) { free_sweep(p); free_bins(p); }
   dfree(p.base); dfree(p.psi); dfree(p.perm); dfree(p.iperm); dfree(p.sframe);
-  dfree(p.interp_items); dfree(p.tile_items); dfree(p.grid_items);
+  dfree(p.interp_items); dfree(p.tile_items); dfree(p.grid_items); dfree(p.gm_waves);
+  p.n_gm_blocks = 0;
   p.n_tile_items = 0; dfree(p.reduce_items); dfree(p.visits); dfree(p.vrec); dfree(p.partial);
   p.n_interp_items = p.n_grid_items = p.n_reduce_items = 0;
   p.n_visits = 0;
@@ -792,6 +793,40 @@ static int sweep_weights(Plan& p, const std::vector<float>& ws) {
   return CGS_OK;
 }
 
+// Waves of the 2D matrix-core scatter (GridArgs::gwaves) over `items` (longest
+// first): gm_shape(C).waves a block, g = 1, 2, 4 .. of them sharing an item so that a wave walks about
+// `share` visits.  g follows from the item and its own frame alone, so a frame's
+// sums do not depend on the other frames of its plan.  share: a frame large
+// enough for eight waves on every SIMD at 64 visits each gives a wave more, up
+// to 256 (256^2 x 32 coils: share 64 / 128 / 176 / 256: 86 / 84 / 81 / 78 us; at
+// 128^2 x 8 coils 15 / 17 / 19 / 23 us).
+static void gm_waves(const Plan& p, const std::vector<GridItem>& items, const std::vector<int64_t>& vcnt,
+                     std::vector<GmWave>& out) {
+  const int64_t tpf = p.tiles_per_frame;
+  const GmShape sh = gm_shape(p.C);
+  const int NW = sh.waves;
+  auto waves_of = [&](const GridItem& it) {
+    const int64_t fv = vcnt[(it.frame + 1) * tpf] - vcnt[it.frame * tpf];
+    const int64_t share = std::min<int64_t>(256, std::max<int64_t>(64, fv * sh.groups / 8192));
+    int g = 1;
+    while (g < NW && share * g < it.vend - it.vbeg) g *= 2;
+    return g;
+  };
+  out.clear();
+  out.reserve(items.size() + 4 * NW);
+  for (size_t q = 0, e; q < items.size(); q = e) {
+    const int g = waves_of(items[q]);
+    for (e = q; e < items.size() && (int)(e - q) < NW / g && waves_of(items[e]) == g; ++e) {
+      const GridItem& it = items[e];
+      const int nv = it.vend - it.vbeg, part = ((nv + g - 1) / g + 7) & ~7;   // multiples of 8 visits
+      for (int j = 0; j < g; ++j)
+        out.push_back(GmWave{it.frame, it.tile, it.vbeg + std::min(nv, j * part),
+                             it.vbeg + std::min(nv, (j + 1) * part), it.slot, g, j, 0});
+    }
+    while (out.size() % NW) out.push_back(GmWave{-1, 0, 0, 0, -1, g, (int)(out.size() % g), 0});
+  }
+}
+
 // sweep: also (re)build the line-sweep tables, which depend on the trajectory
 // only (not on the visit-list chunking the autotuner varies)
 static int build_samples(Plan& p, const float* k, bool sweep = true) {
@@ -915,34 +950,62 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
     std::vector<int64_t> pos(vcnt.begin(), vcnt.end() - 1);
     for_visits([&](int64_t kk, int64_t s) { vis[pos[kk]++] = (int)s; });
   }
-  // visit records: sample id, offsets of the footprint in the tile, in-tile tap ranges
+  // visit records: sample id, offsets of the footprint in the tile, in-tile tap
+  // ranges.  2D lists are sorted by the axis-1 offset (stable), so that runs of
+  // visits meet the same rows of the tile (k_grid_mfma leaves the others out).
   std::vector<int4> vrec((size_t)nvis);
-  for (int64_t kk = 0; kk < nkeys; ++kk) {
-    const int t = (int)(kk % tpf);
-    const int tt[3] = {t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1])};
-    int ts[3], te[3];
-    for (int a = 0; a < 3; ++a) {
-      ts[a] = tt[a] * T;
-      te[a] = (a < d) ? std::min(T, p.n[a] - ts[a]) : 1;
-    }
-    for (int64_t v = vcnt[kk]; v < vcnt[kk + 1]; ++v) {
-      const int s = vis[v];
-      int rel[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
-      for (int a = 0; a < d; ++a) {
-        int r = hbase[(int64_t)s * d + a] - ts[a];
-        if (r < 0) r += p.n[a];
-        if (r >= te[a]) r -= p.n[a];
-        rel[a] = r;
-        lo[a] = std::max(0, -r);
-        hi[a] = std::min(taps, te[a] - r);
+  {
+    const int nthr = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    auto tiles = [&](int th) {
+      std::vector<int4> tmp;
+      // thread th takes the tiles of its share of the visits
+      const int64_t k0 = std::lower_bound(vcnt.begin(), vcnt.end() - 1, nvis * th / nthr) - vcnt.begin();
+      const int64_t k1 = th + 1 == nthr ? nkeys
+                                        : std::lower_bound(vcnt.begin(), vcnt.end() - 1, nvis * (th + 1) / nthr) - vcnt.begin();
+      for (int64_t kk = k0; kk < k1; ++kk) {
+        const int t = (int)(kk % tpf);
+        const int tt[3] = {t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1])};
+        int ts[3], te[3];
+        for (int a = 0; a < 3; ++a) {
+          ts[a] = tt[a] * T;
+          te[a] = (a < d) ? std::min(T, p.n[a] - ts[a]) : 1;
+        }
+        for (int64_t v = vcnt[kk]; v < vcnt[kk + 1]; ++v) {
+          const int s = vis[v];
+          int rel[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, hi[3] = {1, 1, 1};
+          for (int a = 0; a < d; ++a) {
+            int r = hbase[(int64_t)s * d + a] - ts[a];
+            if (r < 0) r += p.n[a];
+            if (r >= te[a]) r -= p.n[a];
+            rel[a] = r;
+            lo[a] = std::max(0, -r);
+            hi[a] = std::min(taps, te[a] - r);
+          }
+          int4 rc;
+          rc.x = s;
+          rc.y = (int)(((uint32_t)rel[0] & 0xffffu) | ((uint32_t)rel[1] << 16));
+          rc.z = (int)((uint32_t)lo[0] | ((uint32_t)hi[0] << 8) | ((uint32_t)lo[1] << 16) | ((uint32_t)hi[1] << 24));
+          rc.w = (d == 3) ? (int)(((uint32_t)rel[2] & 0xffffu) | ((uint32_t)lo[2] << 16) | ((uint32_t)hi[2] << 24)) : 0;
+          vrec[v] = rc;
+        }
+        if (d == 2 && vcnt[kk + 1] - vcnt[kk] > 1) {   // counting sort by rel1 in (-taps, T)
+          const int nc = T + taps;   // (tiles wider than 69 cells stay unsorted)
+          int64_t pos[80] = {0};
+          const int4* src = vrec.data() + vcnt[kk];
+          const int64_t n = vcnt[kk + 1] - vcnt[kk];
+          tmp.assign(src, src + n);
+          if (nc + 1 <= (int)(sizeof(pos) / sizeof(pos[0]))) {
+            for (const int4& r : tmp) pos[(r.y >> 16) + taps + 1]++;
+            for (int q = 0; q < nc; ++q) pos[q + 1] += pos[q];
+            for (const int4& r : tmp) vrec[vcnt[kk] + pos[(r.y >> 16) + taps]++] = r;
+          }
+        }
       }
-      int4 rc;
-      rc.x = s;
-      rc.y = (int)(((uint32_t)rel[0] & 0xffffu) | ((uint32_t)rel[1] << 16));
-      rc.z = (int)((uint32_t)lo[0] | ((uint32_t)hi[0] << 8) | ((uint32_t)lo[1] << 16) | ((uint32_t)hi[1] << 24));
-      rc.w = (d == 3) ? (int)(((uint32_t)rel[2] & 0xffffu) | ((uint32_t)lo[2] << 16) | ((uint32_t)hi[2] << 24)) : 0;
-      vrec[v] = rc;
-    }
+    };
+    std::vector<std::thread> th;
+    for (int t = 1; t < nthr; ++t) th.emplace_back(tiles, t);
+    tiles(0);
+    for (auto& x : th) x.join();
   }
   std::vector<GridItem> gitems;
   std::vector<ReduceItem> ritems;
@@ -966,6 +1029,8 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
   // longest items first
   std::stable_sort(gitems.begin(), gitems.end(),
                    [](const GridItem& x, const GridItem& y) { return (x.vend - x.vbeg) > (y.vend - y.vbeg); });
+  std::vector<GmWave> gmw;
+  if (d == 2 && T == 8) gm_waves(p, gitems, vcnt, gmw);
 
   free_samples(p, sweep);
   CHK(dalloc(&p.base, hbase.size()));
@@ -979,6 +1044,7 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
     HIPCHK(hipMemcpy(p.tile_items, titems.data(), sizeof(int4) * titems.size(), hipMemcpyHostToDevice));
   p.n_tile_items = (int)titems.size();
   CHK(dalloc(&p.grid_items, gitems.size()));
+  CHK(dalloc(&p.gm_waves, gmw.size()));
   CHK(dalloc(&p.reduce_items, ritems.size()));
   CHK(dalloc(&p.visits, vis.size()));
   CHK(dalloc(&p.vrec, vrec.size()));
@@ -998,6 +1064,8 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
     HIPCHK(hipMemcpy(p.interp_items, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice));
   if (!gitems.empty())
     HIPCHK(hipMemcpy(p.grid_items, gitems.data(), sizeof(GridItem) * gitems.size(), hipMemcpyHostToDevice));
+  if (!gmw.empty())
+    HIPCHK(hipMemcpy(p.gm_waves, gmw.data(), sizeof(GmWave) * gmw.size(), hipMemcpyHostToDevice));
   if (!ritems.empty())
     HIPCHK(hipMemcpy(p.reduce_items, ritems.data(), sizeof(ReduceItem) * ritems.size(), hipMemcpyHostToDevice));
   if (!vis.empty()) HIPCHK(hipMemcpy(p.visits, vis.data(), sizeof(int) * vis.size(), hipMemcpyHostToDevice));
@@ -1005,6 +1073,7 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
   if (sweep) CHK(build_bins(p, hbase, hpsi, hframe));
   p.n_interp_items = (int)items.size();
   p.n_grid_items = (int)gitems.size();
+  p.n_gm_blocks = (int)(gmw.size() / gm_shape(p.C).waves);
   p.n_reduce_items = (int)ritems.size();
   p.n_visits = nvis;
   p.n_slots = slots;
@@ -1322,7 +1391,7 @@ static int create_plan(Plan& p, int d, const int* N, int64_t Mtot, double sigma,
   // 72-74 us for one coil a lane); 3D: (sample, plane, tap parity) where taps = 8, T = 8
   p.interp_lanes = (d == 2) ? 4 : 2;
   p.tile_item_max = (d == 3) ? 2048 : 128;
-  p.visits_per_item = (d == 3) ? 4096 : 512;
+  p.visits_per_item = (d == 3) ? 4096 : 1024;   // 2D: shared by the waves of a block
   p.grid_cgr = (C <= 8) ? 8 : 16;
   // shape overrides for tuning sweeps (tile side must be a multiple of 8)
   if (const char* e = std::getenv("CGS_TILE")) {
