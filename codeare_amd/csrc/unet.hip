@@ -61,7 +61,7 @@ __device__ __forceinline__ bf16x8 as_bf8(uint4 v) { return __builtin_bit_cast(bf
 struct ConvArgs {
   const bf16* A;
   const bf16* B;
-  const bf16* Wt;     // [9][Cout][Cin]
+  const uint4* Wt;    // operand order, see k_wprep
   const float* bias;  // [Cout] or null
   bf16* out0;
   bf16* out1;
@@ -71,144 +71,186 @@ struct ConvArgs {
   int relu;
 };
 
-// Block: 4 waves; tile TR x TW pixels x BC output channels; each wave owns
-// 64 pixels (two 32-pixel MFMA rows) x 32 channels.  K is walked in chunks of
-// 32 input channels over all 9 taps, staged through LDS.
-template <int TR, int TW, int BC>
-__global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a) {
-  constexpr int KC = 32;
-  constexpr int HS = KC + 8;            // halves per halo position (16 B pad)
-  constexpr int WS = KC + 8;            // halves per weight row
-  constexpr int HP = (TR + 2) * (TW + 2);
-  constexpr int NWP = TR * TW / 64;     // pixel groups
-  static_assert(NWP * (BC / 32) == 4, "tile must give 4 waves");
-  __shared__ __attribute__((aligned(16))) bf16 hal[HP * HS];
-  __shared__ __attribute__((aligned(16))) bf16 wl[9 * BC * WS];
+// Block: 4 waves; tile 8 PW x 16 pixels x 32 CW output channels; each wave owns
+// PW 32-pixel rows of products (2 image rows of 16) x CW 32-channel columns.  K
+// is walked in chunks of KC input channels (32; 16 for the packed network input),
+// within a chunk over the 9 taps, then over steps of 16 channels: one order of
+// sums for every tile shape.  Per chunk the input halo and the weights go through
+// LDS; the next chunk's loads are in flight while the current one is multiplied.
+// The weights come in operand order (k_wprep), so their staging is a linear copy
+// and their reads are conflict-free; a halo position takes 80 bytes, which puts
+// 16 neighbours on 16 different 16-byte banks.  Products are weights x pixels,
+// D[channel][pixel]: a lane holds one pixel's channels in runs of four, and one
+// swap of the wave's halves makes its stores 16 bytes.
+//
+// What bounds it: at a batch of 16 images of 256^2 the matrix work and, in the
+// 32-channel level, the activations' traffic (665 TFLOP/s forward, 602 input
+// gradient over the 14 layers; 219 with blocks that loaded a chunk, waited and
+// multiplied, weights staged in rows and 2-byte stores); at one image the few
+// blocks' walk over the chunks (14 layers 411 -> 110 us).
+constexpr int kHaloStride = 40;   // halves per halo position (32 channels + 16 bytes)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf2(float x, float y) {   // round to nearest even
+  const f32x2 v = {x, y};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+// barrier for data passed through LDS: does not wait for global loads in flight
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
-  const int Cin = a.Ca + a.Cb;
-  const int tiles_x = a.W / TW, tiles_y = a.H / TR;
+template <int PW, int CW, int KC>
+__global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a) {
+  constexpr int TR = 8 * PW, HP = (TR + 2) * 18, KS = KC / 16, G = KC / 8;
+  constexpr int NH = (HP * G + 255) / 256;             // halo units (16 bytes) per thread
+  constexpr int WU = 9 * KS * CW * 64;                 // weight units per chunk
+  constexpr int NW = (WU + 255) / 256;
+  __shared__ __attribute__((aligned(16))) bf16 hal[HP * kHaloStride];
+  __shared__ u32x4 wl[WU];
+
+  const int Cin = a.Ca + a.Cb, nct = a.Cout / 32;
+  const int tiles_x = a.W / 16, tiles_y = a.H / TR;
   int t = blockIdx.x;
-  const int tx0 = (t % tiles_x) * TW;
+  const int tx0 = (t % tiles_x) * 16;
   t /= tiles_x;
   const int ty0 = (t % tiles_y) * TR;
   const int b = t / tiles_y;
-  const int co0 = blockIdx.y * BC;
+  const int ct0 = blockIdx.y * CW;                     // first 32-channel tile of the block
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wp = w % NWP, wc = w / NWP;
   const int row = lane & 31, kh = lane >> 5;
   const int Hh = a.H >> 1, Wh = a.W >> 1;
 
-  // pixel positions of this lane's two A rows
-  int hpos[2];
+  // this thread's halo units: pixel index at full and at half resolution (0 where
+  // outside the image: loaded and dropped)
+  int pixA[NH], pixB[NH];
+  unsigned inside = 0;
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int p = wp * 64 + s * 32 + row;
-    hpos[s] = (p / TW) * (TW + 2) + (p % TW);
+  for (int u = 0; u < NH; ++u) {
+    const int pos = (u * 256 + tid) / G;
+    const int hy = pos / 18, hx = pos - hy * 18;
+    const int y = ty0 + hy - 1, x = tx0 + hx - 1;
+    const bool ok = pos < HP && y >= 0 && y < a.H && x >= 0 && x < a.W;
+    inside |= (unsigned)ok << u;
+    pixA[u] = ok ? (b * a.H + y) * a.W + x : 0;
+    pixB[u] = ok && a.Cb ? (b * Hh + (y >> 1)) * Wh + (x >> 1) : 0;
   }
+  const int grp8 = (tid % G) * 8;                      // (256 is a multiple of G: the same for every unit)
 
-  f32x16 acc[2];
+  u32x4 hv[NH], wv[NW];
+  auto load_chunk = [&](int c0) {
+    const bool inA = c0 < a.Ca;
+    const bf16* src = inA ? a.A + c0 + grp8 : a.B + (c0 - a.Ca) + grp8;
+    const int st = inA ? a.Ca : a.Cb;
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
+    for (int u = 0; u < NH; ++u)
+      hv[u] = *reinterpret_cast<const u32x4*>(src + (size_t)(unsigned)(inA ? pixA[u] : pixB[u]) * (unsigned)st);
+    // operand order: [step][channel tile][lane], step = (chunk * 9 + tap) * KS + ks
+    const u32x4* ws = reinterpret_cast<const u32x4*>(a.Wt) + ((size_t)(c0 / KC) * 9 * KS * nct + ct0) * 64;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[s][r] = 0.f;
+    for (int u = 0; u < NW; ++u) {
+      const int idx = min(u * 256 + tid, WU - 1);
+      wv[u] = ws[(size_t)(idx / (CW * 64)) * nct * 64 + idx % (CW * 64)];
+    }
+  };
+  auto store_chunk = [&]() {
+#pragma unroll
+    for (int u = 0; u < NH; ++u) {
+      const int pos = (u * 256 + tid) / G;
+      const bool ok = (inside >> u) & 1u;
+      const u32x4 v = ok ? hv[u] : u32x4{0, 0, 0, 0};
+      if (pos < HP) *reinterpret_cast<u32x4*>(&hal[pos * kHaloStride + grp8]) = v;
+    }
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+      if (u * 256 + tid < WU) wl[u * 256 + tid] = wv[u];
+  };
 
+  f32x16 acc[PW][CW];
+#pragma unroll
+  for (int s = 0; s < PW; ++s)
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[s][c][r] = 0.f;
+  const bf16* hp = hal + ((w * 2 * PW + (row >> 4)) * 18 + (row & 15)) * kHaloStride + kh * 8;
+
+  load_chunk(0);
   for (int c0 = 0; c0 < Cin; c0 += KC) {
-    const int kc = min(KC, Cin - c0);   // 16 or 32
-    const int g = kc >> 3;
-    __syncthreads();
-    // ---- stage the input halo: HP positions x g groups of 8 channels
-    {
-      const int total = HP * g;
-      for (int base = 0; base < total; base += 256 * 4) {
-        uint4 v[4];
-        int dst[4];
+    if (c0) lds_sync();                                // the chunk before is consumed
+    store_chunk();
+    if (c0 + KC < Cin) load_chunk(c0 + KC);
+    lds_sync();
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int idx = base + u * 256 + tid;
-          dst[u] = -1;
-          v[u] = make_uint4(0, 0, 0, 0);
-          if (idx < total) {
-            const int pos = idx / g, grp = idx - pos * g;
-            const int hy = pos / (TW + 2), hx = pos - hy * (TW + 2);
-            const int y = ty0 + hy - 1, x = tx0 + hx - 1;
-            const int ci = c0 + grp * 8;
-            dst[u] = pos * HS + grp * 8;
-            if (y >= 0 && y < a.H && x >= 0 && x < a.W) {
-              const bf16* src;
-              if (ci < a.Ca)
-                src = a.A + ((size_t)(b * a.H + y) * a.W + x) * a.Ca + ci;
-              else
-                src = a.B + ((size_t)(b * Hh + (y >> 1)) * Wh + (x >> 1)) * a.Cb + (ci - a.Ca);
-              v[u] = *reinterpret_cast<const uint4*>(src);
-            }
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (dst[u] >= 0) *reinterpret_cast<uint4*>(&hal[dst[u]]) = v[u];
-      }
-    }
-    // ---- stage the weights: 9 taps x BC channels x g groups
-    {
-      const int total = 9 * BC * g;
-      for (int base = 0; base < total; base += 256 * 4) {
-        uint4 v[4];
-        int dst[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int idx = base + u * 256 + tid;
-          dst[u] = -1;
-          if (idx < total) {
-            const int grp = idx % g, rc = idx / g;   // rc = tap*BC + co
-            const int tap = rc / BC, co = rc - tap * BC;
-            dst[u] = rc * WS + grp * 8;
-            v[u] = *reinterpret_cast<const uint4*>(a.Wt + ((size_t)tap * a.Cout + co0 + co) * Cin + c0 + grp * 8);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (dst[u] >= 0) *reinterpret_cast<uint4*>(&wl[dst[u]]) = v[u];
-      }
-    }
-    __syncthreads();
-    // ---- MFMA over 9 taps x kc/16 steps
-#pragma unroll 1
     for (int tap = 0; tap < 9; ++tap) {
-      const int dy = tap / 3, dx = tap - dy * 3;
-      const int shift = dy * (TW + 2) + dx;
-      for (int ks = 0; ks < (kc >> 4); ++ks) {
-        const int koff = ks * 16 + kh * 8;
-        const bf16x8 bv = as_bf8(*reinterpret_cast<const uint4*>(&wl[(tap * BC + wc * 32 + row) * WS + koff]));
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          const bf16x8 av = as_bf8(*reinterpret_cast<const uint4*>(&hal[(hpos[s] + shift) * HS + koff]));
-          acc[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[s], 0, 0, 0);
+      for (int ks = 0; ks < KS; ++ks) {
+        bf16x8 wf[CW];
+#pragma unroll
+        for (int c = 0; c < CW; ++c) wf[c] = __builtin_bit_cast(bf16x8, wl[((tap * KS + ks) * CW + c) * 64 + lane]);
+#pragma unroll
+        for (int s = 0; s < PW; ++s) {
+          const bf16x8 pf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+              hp + ((2 * s + tap / 3) * 18 + tap % 3) * kHaloStride + ks * 16));
+#pragma unroll
+          for (int c = 0; c < CW; ++c) acc[s][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[c], pf, acc[s][c], 0, 0, 0);
         }
       }
     }
   }
 
-  // ---- epilogue: D[row=pixel][col=channel]; lane holds col lane&31 and
-  // rows 8*(r/4) + 4*(lane/32) + (r%4)
-  const int co = co0 + wc * 32 + (lane & 31);
-  const float bv = a.bias ? a.bias[co] : 0.f;
+  // ---- epilogue: lane holds pixel `row`, register r channel 8 (r / 4) + 4 kh + r % 4
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
+  for (int c = 0; c < CW; ++c) {
+    const int co = (ct0 + c) * 32;
+    const bool first = co < a.split;                   // (split is a multiple of 32)
+    bf16* out = first ? a.out0 + co : a.out1 + (co - a.split);
+    const bf16* mask = first && a.mask0 ? a.mask0 + co : nullptr;
+    const int st = first ? a.split : a.Cout - a.split;
+    float bias[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int p = wp * 64 + s * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-      const int y = ty0 + p / TW, x = tx0 + p % TW;
+    for (int r = 0; r < 16; ++r) bias[r] = a.bias ? a.bias[co + 8 * (r >> 2) + 4 * kh + (r & 3)] : 0.f;
+#pragma unroll
+    for (int s = 0; s < PW; ++s) {
+      const int y = ty0 + w * 2 * PW + 2 * s + (row >> 4), x = tx0 + (row & 15);
       const size_t pix = (size_t)(b * a.H + y) * a.W + x;
-      float v = acc[s][r] + bv;
-      if (a.relu) v = fmaxf(v, 0.f);
-      if (co < a.split) {
-        const size_t o = pix * a.split + co;
-        if (a.mask0 && !(bf2f(a.mask0[o]) > 0.f)) v = 0.f;
-        a.out0[o] = f2bf(v);
-      } else {
-        a.out1[pix * (a.Cout - a.split) + (co - a.split)] = f2bf(v);
+      uint32_t d[4][2];                                // quad q: channels 8 q + 4 kh .. + 3
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc[s][c][4 * q + e] + bias[4 * q + e];
+          if (a.relu) v[e] = fmaxf(v[e], 0.f);
+        }
+        d[q][0] = pack_bf2(v[0], v[1]);
+        d[q][1] = pack_bf2(v[2], v[3]);
+      }
+      // halves of the wave swap: lanes 0..31 end with channels 0..15 of their
+      // pixel, lanes 32..63 with channels 16..31
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        uint4 v;
+        const auto s0 = __builtin_amdgcn_permlane32_swap(d[q][0], d[q + 2][0], false, false);
+        const auto s1 = __builtin_amdgcn_permlane32_swap(d[q][1], d[q + 2][1], false, false);
+        v = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        const int ch = 16 * kh + 8 * q;
+        if (mask) {
+          const uint4 m = *reinterpret_cast<const uint4*>(mask + pix * st + ch);
+          auto keep = [](uint32_t x, uint32_t g) {     // halves of x where the bf16 halves of g are > 0
+            const uint32_t lo = (int16_t)(g & 0xffffu) > 0 ? 0xffffu : 0u;
+            const uint32_t hi = (int32_t)g >= 0x10000 ? 0xffff0000u : 0u;
+            return x & (lo | hi);
+          };
+          v = make_uint4(keep(v.x, m.x), keep(v.y, m.y), keep(v.z, m.z), keep(v.w, m.w));
+        }
+        *reinterpret_cast<uint4*>(out + pix * st + ch) = v;
       }
     }
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -531,8 +573,17 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   }
 }
 
-// BF16 working copies of one conv layer: Wf[tap][co][ci] and the flipped,
-// transposed Wb[8 - tap][ci][co]
+// BF16 working copies of one conv layer in the order k_conv3x3 stages them:
+// [step][32-channel output tile][lane][8], step = (chunk * 9 + tap) * KS + ks with
+// chunks of KC = 16 KS input channels, lane = output channel + 32 kh holding input
+// channels chunk KC + 16 ks + 8 kh + 0..7.  wb: the same of the flipped, transposed
+// weights W'[8 - tap][ci][co] (the input-gradient pass), null where no pass reads it.
+__device__ __forceinline__ size_t operand_index(int tap, int co, int ci, int Cout, int Cin) {
+  const int KS = Cin % 32 ? 1 : 2, KC = 16 * KS;
+  const int chunk = ci / KC, ks = (ci % KC) / 16, kh = (ci % 16) / 8;
+  const size_t step = ((size_t)chunk * 9 + tap) * KS + ks;
+  return ((step * (Cout / 32) + co / 32) * 64 + (co % 32) + 32 * kh) * 8 + ci % 8;
+}
 __global__ void k_wprep(const float* __restrict__ wm, bf16* __restrict__ wf, bf16* __restrict__ wb, int Cout, int Cin) {
   const size_t n = (size_t)9 * Cout * Cin;
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
@@ -540,8 +591,8 @@ __global__ void k_wprep(const float* __restrict__ wm, bf16* __restrict__ wf, bf1
     const size_t t = i / Cin;
     const int co = t % Cout, tap = t / Cout;
     const bf16 h = f2bf(wm[i]);
-    wf[i] = h;
-    wb[((size_t)(8 - tap) * Cin + ci) * Cout + co] = h;
+    wf[operand_index(tap, co, ci, Cout, Cin)] = h;
+    if (wb) wb[operand_index(8 - tap, ci, co, Cin, Cout)] = h;
   }
 }
 
@@ -644,24 +695,34 @@ struct Timer {
   }
 };
 
-// forward or input-gradient convolution launch
+// forward or input-gradient convolution launch: the largest tile (pixels x
+// channels) that still gives every CU two blocks, else the one with most blocks
+// (asking for one or four blocks a CU measured the same within 3 %)
+template <int PW, int CW>
+void conv_go(cgs_unet_s& n, const ConvArgs& a) {
+  const dim3 g((unsigned)((a.W / 16) * (a.H / (8 * PW)) * a.batch), (unsigned)(a.Cout / (32 * CW)));
+  if ((a.Ca + a.Cb) % 32) hipLaunchKernelGGL((k_conv3x3<PW, CW, 16>), g, dim3(256), 0, n.stream, a);
+  else hipLaunchKernelGGL((k_conv3x3<PW, CW, 32>), g, dim3(256), 0, n.stream, a);
+}
+
 int conv_launch(cgs_unet_s& n, const ConvArgs& a, int slot) {
   const int Cin = a.Ca + a.Cb;
-  if (a.Cout % 32 || Cin % 16 || a.Ca % 8 || a.Cb % 8) {
-    cgs::set_error("conv channel counts must be multiples of 32 (out) and 16 (in)");
+  // (inputs: 16 channels, or chunks of 32 that lie in one of the two tensors)
+  if (a.Cout % 32 || (Cin != 16 && (a.Ca % 32 || a.Cb % 32))) {
+    cgs::set_error("conv channel counts must be multiples of 32 (or a 16-channel input)");
     return CGS_ERR_UNSUPPORTED;
   }
-  Timer tm(n, slot, 2.0 * 9.0 * Cin * a.Cout * (double)a.H * a.W * a.batch);
-  if (a.Cout % 64 == 0 && a.W % 16 == 0 && a.H % 8 == 0) {
-    dim3 g((a.W / 16) * (a.H / 8) * a.batch, a.Cout / 64);
-    hipLaunchKernelGGL((k_conv3x3<8, 16, 64>), g, dim3(256), 0, n.stream, a);
-  } else if (a.W % 16 == 0 && a.H % 16 == 0) {
-    dim3 g((a.W / 16) * (a.H / 16) * a.batch, a.Cout / 32);
-    hipLaunchKernelGGL((k_conv3x3<16, 16, 32>), g, dim3(256), 0, n.stream, a);
-  } else {
+  if (a.W % 16 || a.H % 16) {
     cgs::set_error("conv tile does not divide the image");
     return CGS_ERR_UNSUPPORTED;
   }
+  Timer tm(n, slot, 2.0 * 9.0 * Cin * a.Cout * (double)a.H * a.W * a.batch);
+  const long long px = (long long)a.H * a.W * a.batch, ct = a.Cout / 32;
+  constexpr long long need = 512;
+  const bool even = ct % 2 == 0;
+  if (even && px / 256 * (ct / 2) >= need) conv_go<2, 2>(n, a);
+  else if (px / 256 * ct >= need) conv_go<2, 1>(n, a);
+  else conv_go<1, 1>(n, a);
   UCHK(hipGetLastError());
   return CGS_OK;
 }
@@ -715,7 +776,7 @@ int prep_weights(cgs_unet_s& n) {
     const int Cin = c.ca + c.cb;
     const size_t nw = (size_t)9 * c.cout * Cin;
     hipLaunchKernelGGL(k_wprep, dim3(grid_for(nw)), dim3(256), 0, n.stream, (const float*)(n.params + c.w_off), c.wf,
-                       c.wb, c.cout, Cin);
+                       Cin % 32 ? nullptr : c.wb, c.cout, Cin);
     UCHK(hipGetLastError());
   }
   return CGS_OK;
@@ -745,9 +806,9 @@ int forward(cgs_unet_s& n, const float2* x, float2* y, const float2* tgt, int ba
     const int H = n.H >> l, W = n.W >> l, C = level_ch(n, l);
     const Conv& ca = n.convs[2 * l];
     const Conv& cb = n.convs[2 * l + 1];
-    RCHK(conv_launch(n, ConvArgs{in, nullptr, ca.wf, n.params + ca.b_off, n.act_a[l], nullptr, nullptr, cin, 0, C, C, H, W,
+    RCHK(conv_launch(n, ConvArgs{in, nullptr, (const uint4*)ca.wf, n.params + ca.b_off, n.act_a[l], nullptr, nullptr, cin, 0, C, C, H, W,
                                  batch, 1}, 0));
-    RCHK(conv_launch(n, ConvArgs{n.act_a[l], nullptr, cb.wf, n.params + cb.b_off, n.act_s[l], nullptr, nullptr, C, 0, C, C,
+    RCHK(conv_launch(n, ConvArgs{n.act_a[l], nullptr, (const uint4*)cb.wf, n.params + cb.b_off, n.act_s[l], nullptr, nullptr, C, 0, C, C,
                                  H, W, batch, 1}, 0));
     if (l < L - 1) {
       Timer tm(n, 6, 0);
@@ -765,9 +826,9 @@ int forward(cgs_unet_s& n, const float2* x, float2* y, const float2* tgt, int ba
     const Conv& da = n.convs[2 * L + 2 * (L - 2 - l)];
     const Conv& db = n.convs[2 * L + 2 * (L - 2 - l) + 1];
     const bf16* below = (l + 1 == L - 1) ? n.act_s[L - 1] : n.act_o[l + 1];
-    RCHK(conv_launch(n, ConvArgs{n.act_s[l], below, da.wf, n.params + da.b_off, n.act_u[l], nullptr, nullptr, C, 2 * C, C,
+    RCHK(conv_launch(n, ConvArgs{n.act_s[l], below, (const uint4*)da.wf, n.params + da.b_off, n.act_u[l], nullptr, nullptr, C, 2 * C, C,
                                  C, H, W, batch, 1}, 0));
-    RCHK(conv_launch(n, ConvArgs{n.act_u[l], nullptr, db.wf, n.params + db.b_off, n.act_o[l], nullptr, nullptr, C, 0, C, C,
+    RCHK(conv_launch(n, ConvArgs{n.act_u[l], nullptr, (const uint4*)db.wf, n.params + db.b_off, n.act_o[l], nullptr, nullptr, C, 0, C, C,
                                  H, W, batch, 1}, 0));
   }
   {
@@ -817,11 +878,11 @@ int backward(cgs_unet_s& n, int batch) {
     bf16* g_below = (l + 1 == L - 1) ? n.g_s[L - 1] : n.g_o[l + 1];
     // conv db: X = u_l, dY = g_o[l]
     RCHK(wgrad_launch(n, n.g_o[l], n.act_u[l], nullptr, C, 0, C, H, W, batch, n.grads + db.w_off, n.grads + db.b_off));
-    RCHK(conv_launch(n, ConvArgs{n.g_o[l], nullptr, db.wb, nullptr, n.g_u[l], nullptr, n.act_u[l], C, 0, C, C, H, W, batch,
+    RCHK(conv_launch(n, ConvArgs{n.g_o[l], nullptr, (const uint4*)db.wb, nullptr, n.g_u[l], nullptr, n.act_u[l], C, 0, C, C, H, W, batch,
                                  0}, 2));
     // conv da: X = (s_l | up(below)), dY = g_u[l]
     RCHK(wgrad_launch(n, n.g_u[l], n.act_s[l], below, C, 2 * C, C, H, W, batch, n.grads + da.w_off, n.grads + da.b_off));
-    RCHK(conv_launch(n, ConvArgs{n.g_u[l], nullptr, da.wb, nullptr, n.g_s[l], n.g_up, n.act_s[l], C, 0, 3 * C, C, H, W,
+    RCHK(conv_launch(n, ConvArgs{n.g_u[l], nullptr, (const uint4*)da.wb, nullptr, n.g_s[l], n.g_up, n.act_s[l], C, 0, 3 * C, C, H, W,
                                  batch, 0}, 2));
     {
       Timer tm(n, 6, 0);
@@ -839,12 +900,12 @@ int backward(cgs_unet_s& n, int batch) {
     const bf16* in = l ? n.act_p[l - 1] : n.xin;
     const int cin = l ? level_ch(n, l - 1) : 16;
     RCHK(wgrad_launch(n, n.g_s[l], n.act_a[l], nullptr, C, 0, C, H, W, batch, n.grads + cb.w_off, n.grads + cb.b_off));
-    RCHK(conv_launch(n, ConvArgs{n.g_s[l], nullptr, cb.wb, nullptr, n.g_a[l], nullptr, n.act_a[l], C, 0, C, C, H, W, batch,
+    RCHK(conv_launch(n, ConvArgs{n.g_s[l], nullptr, (const uint4*)cb.wb, nullptr, n.g_a[l], nullptr, n.act_a[l], C, 0, C, C, H, W, batch,
                                  0}, 2));
     RCHK(wgrad_launch(n, n.g_a[l], in, nullptr, cin, 0, C, H, W, batch, n.grads + ca.w_off, n.grads + ca.b_off));
     if (l > 0) {
       // gradient at the pooled input (unmasked), then routed into g_s[l-1]
-      RCHK(conv_launch(n, ConvArgs{n.g_a[l], nullptr, ca.wb, nullptr, n.g_p[l - 1], nullptr, nullptr, C, 0, cin, cin, H, W,
+      RCHK(conv_launch(n, ConvArgs{n.g_a[l], nullptr, (const uint4*)ca.wb, nullptr, n.g_p[l - 1], nullptr, nullptr, C, 0, cin, cin, H, W,
                                    batch, 0}, 2));
       Timer tm(n, 6, 0);
       const size_t no = (size_t)batch * H * W * cin;
