@@ -882,144 +882,6 @@ __global__ void __launch_bounds__(512) k_grid_reg3(GridArgs a, const int4* __res
   }
 }
 
-// 3D on the matrix cores: one block of 8 waves per work item, wave w owning
-// plane w of the 8 x 8 x 8 tile as D[64 cells][32 columns] (16 coils, re/im).
-// Visit batches (records, window values, weighted data) are staged once per
-// block; each wave compacts the visits whose footprint meets its plane (ballot
-// and prefix count) and applies them two at a time with v_mfma_f32_32x32x2f32
-// per 32-cell half.  Visits keep their list order within a wave:
-// deterministic, no atomics.
-template <int TAPS>
-__global__ void __launch_bounds__(512) k_grid_mfma3(GridArgs a, const int4* __restrict__ vrec, int nitems) {
-  constexpr int B = 64, NPSI = 3 * TAPS, CC = 16;
-  // one more visit slot, B: a footprint outside every tile with zero data,
-  // for the odd lane of a wave's last pair (so the pair loop has no branch)
-  __shared__ float2 sy[(B + 1) * CC];
-  __shared__ float spsi[(B + 1) * NPSI];
-  __shared__ int4 srec[B + 1];
-  __shared__ unsigned char slist[8][B];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const GridItem it = a.items[blockIdx.x];
-  if (a.fdone && a.fdone[it.frame]) return;   // block-uniform
-  const int cbase = blockIdx.y * CC;
-  const int t0 = it.tile % a.nt0, t1 = (it.tile / a.nt0) % a.nt1, t2 = it.tile / (a.nt0 * a.nt1);
-  const int ts0 = t0 * 8, ts1 = t1 * 8, ts2 = t2 * 8;
-  const int te0 = min(8, a.n0 - ts0), te1 = min(8, a.n1 - ts1), te2 = min(8, a.n2 - ts2);
-  const int i = lane & 31, kk = lane >> 5;
-  const int cx = i & 7, cy0 = i >> 3, cy1 = 4 + (i >> 3);
-  gf32x16 acc0, acc1;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
-  if (tid < CC) sy[B * CC + tid] = make_float2(0.f, 0.f);
-  if (tid < NPSI) spsi[B * NPSI + tid] = 0.f;
-  if (tid == 0) srec[B] = make_int4(0, 0x40004000, 0x4000, 0x4000);
-
-  for (int vb = it.vbeg; vb < it.vend; vb += B) {
-    const int nb = min(B, it.vend - vb);
-    lds_barrier();   // the previous batch is consumed (and the pad slot written)
-    if (tid < nb) srec[tid] = vrec[vb + tid];
-    lds_barrier();
-    {
-      // every load of the batch in flight before the first LDS write
-      constexpr int UP = (B * NPSI + 511) / 512, UY = (B * CC + 511) / 512;
-      float pv[UP];
-      float2 yv[UY];
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int idx = tid + 512 * u;
-        pv[u] = 0.f;
-        if (idx < nb * NPSI) {
-          const int v = idx / NPSI, q = idx - v * NPSI;
-          pv[u] = a.psi[(int64_t)srec[v].x * NPSI + q];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UY; ++u) {
-        const int idx = tid + 512 * u;
-        yv[u] = make_float2(0.f, 0.f);
-        if (idx < nb * CC) {
-          const int v = idx / CC, c = idx - v * CC;
-          if (cbase + c < a.C) {
-            const int smp = srec[v].x;
-            yv[u] = a.y[(int64_t)smp * a.C + cbase + c];
-            if (a.w) { const float ww = a.w[smp]; yv[u].x *= ww; yv[u].y *= ww; }
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UP; ++u) {
-        const int idx = tid + 512 * u;
-        if (idx < nb * NPSI) spsi[idx] = pv[u];
-      }
-#pragma unroll
-      for (int u = 0; u < UY; ++u) {
-        const int idx = tid + 512 * u;
-        if (idx < nb * CC) sy[idx] = yv[u];
-      }
-    }
-    // the visits of this batch whose footprint meets plane w, in list order
-    bool hit = false;
-    if (lane < nb) {
-      const int dz = w - (int)(short)(srec[lane].w & 0xffff);
-      hit = (unsigned)dz < (unsigned)TAPS;
-    }
-    const unsigned long long mask = __ballot(hit);
-    const int cnt = __popcll(mask);
-    if (hit) slist[w][__popcll(mask & ((1ull << lane) - 1ull))] = (unsigned char)lane;
-    lds_barrier();   // staged data and this wave's list are visible
-    for (int p = 0; p < cnt; p += 2) {
-      // branch-free: past cnt the pad slot B (zero data, weights selected to 0)
-      const int v = (p + kk < cnt) ? slist[w][p + kk] : B;
-      const int4 rc = srec[v];
-      const int rel0 = (int)(short)(rc.y & 0xffff), rel1 = (int)(short)(rc.y >> 16);
-      const int dz = w - (int)(short)(rc.w & 0xffff);   // in [0, TAPS) for listed visits
-      const float* ps = spsi + v * NPSI;
-      const int dx = cx - rel0, dy0 = cy0 - rel1, dy1 = cy1 - rel1;
-      const bool okx = (unsigned)dx < (unsigned)TAPS && (unsigned)dz < (unsigned)TAPS;
-      const bool ok0 = okx && (unsigned)dy0 < (unsigned)TAPS, ok1 = okx && (unsigned)dy1 < (unsigned)TAPS;
-      const float px = ps[okx ? dx : 0], pz = ps[2 * TAPS + (okx ? dz : 0)];
-      const float q0 = ps[TAPS + (ok0 ? dy0 : 0)], q1 = ps[TAPS + (ok1 ? dy1 : 0)];
-      const float bv = ((const float*)sy)[v * 2 * CC + i];
-      const float pxz = px * pz;
-      const float w0 = ok0 ? pxz * q0 : 0.f, w1 = ok1 ? pxz * q1 : 0.f;
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(w0, bv, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(w1, bv, acc1, 0, 0, 0);
-    }
-  }
-
-  if (w >= te2) return;
-  const int ncol = 2 * min(CC, a.C - cbase);
-  if (i >= ncol) return;
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int cell = 32 * h + 8 * (r >> 2) + 4 * kk + (r & 3);
-      const int x0 = cell & 7, x1 = cell >> 3;
-      if (x0 >= te0 || x1 >= te1) continue;
-      float* out;
-      if (it.slot < 0) {
-        const int64_t l = (ts0 + x0) + (int64_t)a.n0 * ((ts1 + x1) + (int64_t)a.n1 * (ts2 + w));
-        out = (float*)(a.grid + ((int64_t)it.frame * a.ntot + l) * a.C + cbase);
-      } else {
-        out = (float*)(a.partial + ((int64_t)it.slot * a.tilecells + x0 + 8 * (x1 + 8 * w)) * a.C + cbase);
-      }
-      out[i] = h == 0 ? acc0[r] : acc1[r];
-    }
-}
-
-void launch_grid_mfma3(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s) {
-  if (nitems == 0) return;
-  const dim3 g((unsigned)nitems, (unsigned)((a.C + 15) / 16));
-  switch (a.taps) {
-    case 4: hipLaunchKernelGGL((k_grid_mfma3<4>), g, dim3(512), 0, s, a, vrec, nitems); break;
-    case 6: hipLaunchKernelGGL((k_grid_mfma3<6>), g, dim3(512), 0, s, a, vrec, nitems); break;
-    case 8: hipLaunchKernelGGL((k_grid_mfma3<8>), g, dim3(512), 0, s, a, vrec, nitems); break;
-    case 10: hipLaunchKernelGGL((k_grid_mfma3<10>), g, dim3(512), 0, s, a, vrec, nitems); break;
-    default: break;
-  }
-}
-
 void launch_grid_reg3(const GridArgs& a, const int4* vrec, int cgr, int nitems, int ncgroups, hipStream_t s) {
   if (nitems == 0) return;
   const dim3 g((unsigned)nitems, (unsigned)ncgroups);
@@ -1145,7 +1007,7 @@ __global__ void __launch_bounds__(64 * NW, 4) k_grid_mfma(GridArgs a, const int4
   float4 yv[UY];
   int4 rc = make_int4(0, 0, 0, 0);
   unsigned in_foot = 0, need_next[NH], need[NH];
-  auto load_rec = [&](int vb) { rc = vrec[min(vb + (lane & (B - 1)), v1 - 1)]; };
+  auto load_rec = [&](int vb) { rc = vrec[min((unsigned)vb + (lane & (B - 1)), (unsigned)v1 - 1)]; };
   auto put_rec = [&](int nb) {                   // past the list: a footprint outside every tile
     const int ry = (lane & (B - 1)) < nb ? rc.y : 0x40004000;
     if (lane < B) wrec[lane] = make_int2(rc.x, ry);
@@ -1321,6 +1183,238 @@ void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nblocks, hipStrea
   const GmShape sh = gm_shape(a.C);
   if (sh.waves == 8) grid_mfma_taps<16, 8>(a, vrec, nblocks, sh.groups, s);
   else grid_mfma_taps<32, 4>(a, vrec, nblocks, sh.groups, s);
+}
+
+// ---------------------------------------------------------------------------
+// adjoint B^T on the matrix cores (3D, 8x8x8 tiles): one block of 8 waves per work
+// item, wave w owning plane w of the tile as D[64 cells][columns] with the products
+// and operand layouts of k_grid_mfma (R = 32: 16 coils, R = 16: 8 coils).  Batches of
+// 64 visits are staged once per block, double-buffered with one barrier a batch: a
+// visit's record in LDS is its window values placed on the tile's 8 + 8 + 8 axis
+// cells (density weight in the axis-0 factor) and its data, so a product's weight is
+// px pz q from LDS; the next batch's loads and the records of the one after are in
+// flight meanwhile, branch-free.  Each wave lists the visits whose footprint meets
+// its plane (ballot and prefix count); the list is sorted by the axis-1 offset, so the
+// visits that meet a group of R cells are one range of it and the other products are
+// left out (27 % of them).  Visits keep their order within a wave: deterministic, no
+// atomics.
+//
+// What bounds it: on the 128^3 koosh ball (5.12 M samples, 16 coils) the products left
+// are 2.8 ms of matrix work of 7.4 ms; the waves spend about half their time at the
+// batch's barrier and loads (the planes' visit counts of a batch differ), so the
+// register cap for three blocks a CU pays although it spills ten registers outside the
+// product loop (7.95 ms uncapped, two blocks).  Measured against one staged footprint
+// placed per product, without double buffering (one work item of at most 4096 visits a
+// block in both): 10.2 -> 7.4 ms; 96^3 x 8 coils, 768 000 samples: 1.55 -> 0.60 ms.
+// Not kept: lane reads of the list instead of LDS reads (8.9 ms), items of 512-2048
+// visits (9.6-8.4 ms).
+constexpr int kG3Batch = 64;
+template <int TAPS, int R, bool WIDE>
+__global__ void __launch_bounds__(512, 6) k_grid_mfma3(GridArgs a, const int4* __restrict__ vrec, int ngroups) {
+  constexpr int B = kG3Batch, CC = R / 2, NPSI = 3 * TAPS;
+  constexpr int KV = 64 / R, NH = 64 / R, NR = R == 32 ? 16 : 4;
+  constexpr int VS = 24 + R;                     // floats of a visit's record: weights, data
+  constexpr int UW = B * 24 / 512;
+  constexpr int NY = B * CC / 2;                 // 16-byte data units of a batch (512 or 256)
+  // one more record, B: zeros, for the odd lanes of a wave's last product
+  __shared__ __attribute__((aligned(16))) float sv[2][(B + 1) * VS];
+  __shared__ int4 srec[4][B];
+  __shared__ unsigned short slist[8][B + 4 * KV];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int item = blockIdx.x / ngroups;         // every coil group of an item together: the longest first
+  const GridItem it = a.items[item];
+  if (a.fdone && a.fdone[it.frame]) return;      // block-uniform
+  const int cbase = (blockIdx.x - item * ngroups) * CC;
+  const int t0 = it.tile % a.nt0, t1 = (it.tile / a.nt0) % a.nt1, t2 = it.tile / (a.nt0 * a.nt1);
+  const int ts0 = t0 * 8, ts1 = t1 * 8, ts2 = t2 * 8;
+  const int te0 = min(8, a.n0 - ts0), te1 = min(8, a.n1 - ts1), te2 = min(8, a.n2 - ts2);
+  const int i = lane % R, kk = lane / R;
+  gf32x16 acc32[R == 32 ? NH : 1];
+  gf32x4 acc16[R == 16 ? NH : 1];
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if constexpr (R == 32) acc32[h][r] = 0.f;
+      else acc16[h][r] = 0.f;
+    }
+  if (tid < VS) sv[0][B * VS + tid] = sv[1][B * VS + tid] = 0.f;
+
+  const float* dens = a.w ? a.w : a.psi;
+  const int v0 = it.vbeg, v1 = it.vend;
+  float pv[UW], wt = 1.f;
+  float4 yv;
+  int4 rc = make_int4(0, 0, 0, 0);
+  unsigned in_foot = 0;
+  // wave 0 brings the records; past the list: a footprint outside every tile
+  auto load_rec = [&](int vb) {
+    if (w == 0) rc = vrec[min((unsigned)vb + lane, (unsigned)v1 - 1)];
+  };
+  auto put_rec = [&](int slot, int nb) {
+    if (w == 0) srec[slot][lane] = lane < nb ? rc : make_int4(rc.x, 0x40004000, 0, 0x4000);
+  };
+  auto load_batch = [&](int slot) {
+    in_foot = 0;
+    int dx = 0;                                  // (512 = 8 mod 24: one of the three is on axis 0)
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+      const int idx = tid + 512 * u, v = idx / 24, q = idx - v * 24, ax = q >> 3;
+      const int4 r = srec[slot][v];
+      if (ax == 0) dx = r.x;
+      const int rel = ax == 0 ? (int)(short)(r.y & 0xffff) : ax == 1 ? r.y >> 16 : (int)(short)(r.w & 0xffff);
+      const int t = (q & 7) - rel;
+      in_foot |= (unsigned)((unsigned)t < (unsigned)TAPS) << u;
+      pv[u] = a.psi[(int64_t)r.x * NPSI + ax * TAPS + min(max(t, 0), TAPS - 1)];
+    }
+    wt = dens[dx];
+    if (NY == 512 || tid < NY) {
+      const int v = tid / (CC / 2), c = cbase + 2 * (tid % (CC / 2));
+      const float2* src = a.y + (int64_t)srec[slot][v].x * a.C;   // columns past C are not stored
+      if constexpr (WIDE) {
+        yv = *reinterpret_cast<const float4*>(src + min(c, a.C - 2));
+      } else {
+        const float2 p = src[min(c, a.C - 1)], q = src[min(c + 1, a.C - 1)];
+        yv = make_float4(p.x, p.y, q.x, q.y);
+      }
+    }
+  };
+  auto put_batch = [&](float* buf, int nb) {
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+      const int idx = tid + 512 * u, v = idx / 24, q = idx - v * 24;
+      buf[v * VS + q] = (in_foot >> u) & 1u ? pv[u] * (a.w && q < 8 ? wt : 1.f) : 0.f;
+    }
+    if (NY == 512 || tid < NY) {
+      const int v = tid / (CC / 2);
+      const bool ok = v < nb;
+      *reinterpret_cast<float4*>(buf + v * VS + 24 + 4 * (tid % (CC / 2))) =
+          make_float4(ok ? yv.x : 0.f, ok ? yv.y : 0.f, ok ? yv.z : 0.f, ok ? yv.w : 0.f);
+    }
+  };
+  const int lx = (i & 7), lq = 8 + (i >> 3), lz = 16 + w, ly = 24 + i;   // this lane's floats of a record
+  auto multiply = [&](const float* buf, int slot) {
+    // the visits of this batch whose footprint meets plane w, in list order, and
+    // for each group h the range [s, e) of that list that meets its axis-1 cells
+    const int4 r = srec[slot][lane];
+    const int r1 = r.y >> 16;
+    const bool hit = (unsigned)(w - (int)(short)(r.w & 0xffff)) < (unsigned)TAPS && r1 < 8;
+    const unsigned long long mask = __ballot(hit);
+    const int cnt = __popcll(mask);
+    int s[NH], e[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      s[h] = cnt - __popcll(__ballot(hit && r1 + TAPS > h * (R / 8)));
+      e[h] = __popcll(__ballot(hit && r1 < (h + 1) * (R / 8)));
+    }
+    if (hit) slist[w][__popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)(lane * VS);
+    if (lane < 4 * KV) slist[w][cnt + lane] = (unsigned short)(B * VS);   // zeros past the list
+    wave_lds_order();
+    // the next product's operands are read before the current one's products, the
+    // visit of the one after before that
+    float x, z, b, q[NH], nx, nz, nb, nq[NH];
+    auto read = [&](int off) {
+      const float* rec = buf + off;
+      nx = rec[lx];
+      nz = rec[lz];
+      nb = rec[ly];
+#pragma unroll
+      for (int h = 0; h < NH; ++h) nq[h] = rec[lq + h * (R / 8)];
+    };
+    read(slist[w][kk]);
+    int off = slist[w][KV + kk];
+    for (int p = 0; p < cnt; p += KV) {
+      x = nx; z = nz; b = nb;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) q[h] = nq[h];
+      read(off);
+      off = slist[w][p + 2 * KV + kk];
+      const float xz = x * z;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        if (p + KV <= s[h] || p >= e[h]) continue;
+        const float wgt = xz * q[h];
+        if constexpr (R == 32) acc32[h] = __builtin_amdgcn_mfma_f32_32x32x2f32(wgt, b, acc32[h], 0, 0, 0);
+        else acc16[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wgt, b, acc16[h], 0, 0, 0);
+      }
+    }
+    wave_lds_order();
+  };
+
+  if (v0 < v1) {
+    const int nbat = (v1 - v0 + B - 1) / B;
+    load_rec(v0);
+    put_rec(0, v1 - v0);
+    load_rec(v0 + B);
+    put_rec(1, v1 - v0 - B);
+    lds_barrier();
+    load_batch(0);
+    put_batch(sv[0], v1 - v0);
+    load_rec(v0 + 2 * B);
+    put_rec(2, v1 - v0 - 2 * B);
+    lds_barrier();
+    // batch k: data in sv[k & 1], records of batches k .. k + 2 in srec[j & 3]
+    for (int k = 0; k < nbat; ++k) {
+      const bool more = k + 1 < nbat;
+      if (more) {
+        load_batch((k + 1) & 3);
+        load_rec(v0 + (k + 3) * B);
+      }
+      multiply(sv[k & 1], k & 3);
+      if (more) {
+        put_batch(sv[(k + 1) & 1], v1 - v0 - (k + 1) * B);
+        put_rec((k + 3) & 3, v1 - v0 - (k + 3) * B);
+        lds_barrier();
+      }
+    }
+  }
+
+  // registers 4 q .. 4 q + 3 of group h: axis-0 cells xb .. xb + 3 of axis-1 cell x1
+  if (w >= te2) return;
+  const int ncol = 2 * min(CC, a.C - cbase);
+  if (i >= ncol) return;
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int q = 0; q < NR / 4; ++q) {
+      const int x1 = R == 32 ? 4 * h + q : 2 * h + (kk >> 1);
+      const int xb = R == 32 ? 4 * kk : 4 * (kk & 1);
+      if (x1 >= te1) continue;
+      const int64_t l = it.slot < 0
+          ? (int64_t)it.frame * a.ntot + ts0 + xb + (int64_t)a.n0 * (ts1 + x1 + (int64_t)a.n1 * (ts2 + w))
+          : (int64_t)it.slot * a.tilecells + xb + 8 * (x1 + 8 * w);
+      float* out = (float*)((it.slot < 0 ? a.grid : a.partial) + l * a.C + cbase) + i;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float v;
+        if constexpr (R == 32) v = acc32[h][4 * q + j];
+        else v = acc16[h][j];
+        if (xb + j < te0) out[(int64_t)j * 2 * a.C] = v;
+      }
+    }
+}
+
+template <int R>
+static void grid_mfma3_taps(const GridArgs& a, const int4* vrec, int nitems, int ng, hipStream_t s) {
+  const dim3 g((unsigned)nitems * (unsigned)ng);
+#define CGS_GM3(TP)                                                                                      \
+  do {                                                                                                   \
+    if (a.C % 2 == 0) hipLaunchKernelGGL((k_grid_mfma3<TP, R, true>), g, dim3(512), 0, s, a, vrec, ng);   \
+    else hipLaunchKernelGGL((k_grid_mfma3<TP, R, false>), g, dim3(512), 0, s, a, vrec, ng);               \
+  } while (0)
+  switch (a.taps) {
+    case 4: CGS_GM3(4); break;
+    case 6: CGS_GM3(6); break;
+    case 8: CGS_GM3(8); break;
+    case 10: CGS_GM3(10); break;
+    default: break;
+  }
+#undef CGS_GM3
+}
+
+void launch_grid_mfma3(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s) {
+  if (nitems == 0) return;
+  if (a.C <= 8) grid_mfma3_taps<16>(a, vrec, nitems, 1, s);
+  else grid_mfma3_taps<32>(a, vrec, nitems, (a.C + 15) / 16, s);
 }
 
 size_t grid_atomic_lds(int d, int T, int taps, int CG, int rowstride) {

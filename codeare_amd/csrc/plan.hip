@@ -951,11 +951,12 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
     for_visits([&](int64_t kk, int64_t s) { vis[pos[kk]++] = (int)s; });
   }
   // visit records: sample id, offsets of the footprint in the tile, in-tile tap
-  // ranges.  2D lists are sorted by the axis-1 offset (stable), so that runs of
-  // visits meet the same rows of the tile (k_grid_mfma leaves the others out).
+  // ranges.  Lists are sorted by the axis-1 offset (stable), so that runs of visits
+  // meet the same rows of the tile (the matrix-core scatters leave the others out).
   std::vector<int4> vrec((size_t)nvis);
   {
-    const int nthr = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    // (a thread per 32768 visits: starting one costs about as much as that many records)
+    const int nthr = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(16u, std::thread::hardware_concurrency()), nvis >> 15));
     auto tiles = [&](int th) {
       std::vector<int4> tmp;
       // thread th takes the tiles of its share of the visits
@@ -988,7 +989,7 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
           rc.w = (d == 3) ? (int)(((uint32_t)rel[2] & 0xffffu) | ((uint32_t)lo[2] << 16) | ((uint32_t)hi[2] << 24)) : 0;
           vrec[v] = rc;
         }
-        if (d == 2 && vcnt[kk + 1] - vcnt[kk] > 1) {   // counting sort by rel1 in (-taps, T)
+        if (vcnt[kk + 1] - vcnt[kk] > 1) {   // counting sort by rel1 in (-taps, T)
           const int nc = T + taps;   // (tiles wider than 69 cells stay unsorted)
           int64_t pos[80] = {0};
           const int4* src = vrec.data() + vcnt[kk];

@@ -1,4 +1,4 @@
-"""The 2D matrix-core scatter at the edges of its tiles, coil groups and visit
+"""The matrix-core scatters at the edges of its tiles, coil groups and visit
 lists, against the FP64 oracle's adjoint: coil counts around the 8- and 16-coil
 groups (odd ones without 16-byte loads), every window width, grids whose sides
 are not multiples of the 8-cell tile, lists shared by 1 to 8 waves, split over
@@ -47,4 +47,33 @@ def test_scatter_matches_oracle(cgs, ora, C, m, N, kind):
     e1 = max(rel(a[..., c], O.adjoint(y[:, c])) for c in range(C))
     e2 = rel(P.EH(y), O.EH_true(S, w, y))
     print(f"C={C} m={m} N={N} {kind}: adjoint {e1:.2e}, E^H W {e2:.2e}")
+    assert e1 <= 1e-5 and e2 <= 1e-5
+
+
+@pytest.mark.parametrize("C,m,N,kind", [
+    (1, 3, (16, 16, 16), "dense"), (8, 2, (18, 16, 12), "dense"), (7, 4, (16, 12, 16), "few"),
+    (9, 3, (12, 18, 16), "dense"), (16, 1, (16, 16, 18), "spread"), (17, 3, (16, 16, 16), "spread"),
+])
+def test_scatter_3d_matches_oracle(cgs, ora, C, m, N, kind):
+    """3D: partial tiles on every axis, items split over blocks, batches with few or no
+    visits of a plane.  FP32 sums as above."""
+    rng = np.random.default_rng(7000 + 100 * C + m)
+    M = {"few": 3, "spread": 1500, "dense": 6000}[kind]
+    k = rng.uniform(-0.5, 0.5, size=(3, M))
+    if kind == "dense":
+        k[:, 1000:] *= 0.08
+    k = np.asfortranarray(k.astype(np.float32))
+    w = rng.uniform(0.2, 1.0, M).astype(np.float32)
+    S = rand_img(rng, N + (C,))
+    y = rand_img(rng, (M, C))
+    P = cgs.Plan(N, M, 2.0 if m == 4 else 1.5, m, ncoils=C)
+    P.kspace(k)
+    P.weights(w)
+    P.sensitivities(S)
+    O = ora.NFFT(N, M, 2.0 if m == 4 else 1.5, m)
+    O.kspace(k)
+    a = P.nfft_adjoint(y).reshape(N + (C,), order="F")
+    e1 = max(rel(a[..., c], O.adjoint(y[:, c])) for c in range(C))
+    e2 = rel(P.EH(y), O.EH_true(S, w, y))
+    print(f"3D C={C} m={m} N={N} {kind}: adjoint {e1:.2e}, E^H W {e2:.2e}")
     assert e1 <= 1e-5 and e2 <= 1e-5
