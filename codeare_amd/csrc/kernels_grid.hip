@@ -1694,12 +1694,17 @@ __global__ void __launch_bounds__(NT, NT / 128) k_interp_lds3(SampArgs a, const 
 // values and base cells come from global memory, one address per sample
 // broadcast to its lanes, so only the region sits in LDS.
 template <int TAPS, int NT, int TT, int SPLIT>
-__global__ void __launch_bounds__(NT, NT / 128) k_interp_cs3(SampArgs a, const int4* items, int T_, int nt0,
-                                                             int nt1, int ppad) {
+__global__ void __launch_bounds__(NT, NT / 128) k_interp_cs3(SampArgs a, const int4* items, int nitems, int ngroups,
+                                                             int T_, int nt0, int nt1, int ppad) {
   static_assert(TAPS == 8, "8 planes per sample: one per lane group");
   constexpr int CG = 2, NW = NT / 64, LPS = SPLIT ? 16 : 8, SPW = 64 / LPS;
   extern __shared__ float2 sh[];
-  const int4 it = items[blockIdx.x];            // frame, tile, sbeg, send
+  // the coil pairs of an item one after the other on one XCD (a block's XCD is its
+  // index mod 8): a pair stages 16 of every 128 bytes of the item's region, so the
+  // other pairs find their lines in that XCD's L2
+  const int j = blockIdx.x >> 3, pair = j % ngroups, item = (j / ngroups) * 8 + (blockIdx.x & 7);
+  if (item >= nitems) return;
+  const int4 it = items[item];                  // frame, tile, sbeg, send
   if (a.fdone && a.fdone[it.x]) return;
   const int T = TT > 0 ? TT : T_;
   const int E = T + TAPS - 1;
@@ -1707,7 +1712,7 @@ __global__ void __launch_bounds__(NT, NT / 128) k_interp_cs3(SampArgs a, const i
   const int m = TAPS / 2 - 1;
   const int E3 = E * E * E;
   float2* ext = sh;                                     // [E][PS][2]
-  const int cbase = blockIdx.y * CG;
+  const int cbase = pair * CG;
   const int t0 = it.y % nt0, t1 = (it.y / nt0) % nt1, t2 = it.y / (nt0 * nt1);
   const int org0 = t0 * T - m, org1 = t1 * T - m, org2 = t2 * T - m;
   const int64_t gbase = (int64_t)it.x * a.ntot;
@@ -1835,11 +1840,12 @@ void launch_interp_cs3(const SampArgs& a, const int4* items, int nitems, int T, 
   static const int ppad = [] { const char* e = std::getenv("CGS_INTERP3_PAD"); return e ? std::max(0, std::min(15, std::atoi(e))) : 1; }();
   const size_t E = (size_t)T + a.taps - 1;
   const size_t shm = sizeof(float2) * E * (E * E + (split ? ppad : 0)) * 2;
-  const dim3 g((unsigned)nitems, (unsigned)((a.C + 1) / 2));
+  const int ng = (a.C + 1) / 2;
+  const dim3 g((unsigned)((nitems + 7) / 8 * 8) * (unsigned)ng);
 #define CGS_IC3(NT_, SP_)                                                                                        \
   do {                                                                                                         \
-    if (T == 8) hipLaunchKernelGGL((k_interp_cs3<8, NT_, 8, SP_>), g, dim3(NT_), shm, s, a, items, T, nt0, nt1, ppad); \
-    else hipLaunchKernelGGL((k_interp_cs3<8, NT_, 0, SP_>), g, dim3(NT_), shm, s, a, items, T, nt0, nt1, ppad);        \
+    if (T == 8) hipLaunchKernelGGL((k_interp_cs3<8, NT_, 8, SP_>), g, dim3(NT_), shm, s, a, items, nitems, ng, T, nt0, nt1, ppad); \
+    else hipLaunchKernelGGL((k_interp_cs3<8, NT_, 0, SP_>), g, dim3(NT_), shm, s, a, items, nitems, ng, T, nt0, nt1, ppad);        \
   } while (0)
   if (split) {
     if (threads >= 1024) CGS_IC3(1024, 1);
