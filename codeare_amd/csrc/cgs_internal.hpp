@@ -178,7 +178,9 @@ struct FftArgs {
   int nst, radix[8];
   uint32_t ns_magic[8]; // ceil(2^32 / Ns) of each stage (Ns = product of earlier radices)
   int lb_log2;          // lb = 1 << lb_log2
-  int use_reg;          // register-resident kernel (n = 256 or 512, 16 lines per block)
+  int use_reg;          // register-resident kernel k_fft_r8 (n = 256, 384 or 512, inner >= 16)
+  int use_pt;           // register-resident kernel k_fft_pt
+  int lines_log2;       // k_fft_pt: lanes per row = 1 << lines_log2, 16 >> lines_log2 rows per block
   // fused operations of the first forward / last adjoint pass (axis 0)
   const float2* x;      // image frames (load mode 1)
   const float2* S;      // maps (load mode 1); frame f's maps start at S + f*Sfs
@@ -532,7 +534,9 @@ LaunchEvents& launch_events();
   } while (0)
 
 void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
-bool fft_reg_supported(const FftArgs& a, int ld_mode, int st_mode);
+bool fft_reg_supported(const FftArgs& a);
+bool fft_pt_supported(const FftArgs& a);
+void launch_fft_pt(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
 void launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
 bool toep_pad_crop_supported(int N0, int N1, int C);
 bool toep_conv_supported(int N0, int N1, int C);

@@ -330,6 +330,10 @@ __global__ void __launch_bounds__(kFftThreads) k_fft(FftArgs a) {
 size_t fft_lds_bytes(const FftArgs& a) { return sizeof(float2) * ((size_t)a.lb * a.ldn + a.n); }
 
 void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
+  if (a.use_pt) {
+    launch_fft_pt(a, ld_mode, st_mode, s);
+    return;
+  }
   if (a.use_reg) {
     launch_fft_reg(a, ld_mode, st_mode, s);
     return;

@@ -256,8 +256,17 @@ static bool fft_reg_enabled() {
 }
 
 static void fft_finish(FftArgs& a) {
-  a.use_reg = fft_reg_enabled() && fft_reg_supported(a, 0, 0);
-  a.lb = a.use_reg ? 16 : pick_lb(a.inner, a.n);
+  // k_fft_r8 at 256, 384 and 512 points (why: kernels_fft_reg.hip), k_fft_pt at its
+  // lengths, the LDS kernel k_fft at the others: every stage of k_fft passes
+  // the line through LDS, which costs 2 to 9 times the memory traffic's time
+  // (432-point lines, 12 coils: 22.4 us a pass against 8.8; the Toeplitz
+  // convolution at 576 points, 20 coils: 508 against 31 us)
+  const bool reg = fft_reg_enabled();
+  a.lines_log2 = 0;
+  while ((1 << a.lines_log2) < a.inner && a.lines_log2 < 4) ++a.lines_log2;
+  a.use_reg = reg && fft_reg_supported(a);
+  a.use_pt = reg && !a.use_reg && fft_pt_supported(a);
+  a.lb = (a.use_reg || a.use_pt) ? 16 : pick_lb(a.inner, a.n);
   a.lb_log2 = 0;
   while ((1 << a.lb_log2) < a.lb) ++a.lb_log2;
   a.ldn = a.n + (a.n >> 4) + 1;   // room for the 1-in-16 pad slots of the line layout
@@ -1698,7 +1707,7 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
     if (ld == 4) apply_pupd(p, a, pu);
     if (That) { a.That = That; a.conv_cells = cells; a.pad_in = 1; a.crop_out = 1; }
     fft_finish(a);
-    if (pu && tail_out && p.tail_pp && a.use_reg) {
+    if (pu && tail_out && p.tail_pp && (a.use_reg || (a.use_pt && a.lines_log2 == 4))) {
       if (ld == 4) { a.pp_part = p.tail_pp; ++tail_parts; }
       if (st == 2) { a.pq_part = p.tail_pq; a.pdot = pu->pnew; ++tail_parts; }
     }
