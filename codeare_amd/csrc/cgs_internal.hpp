@@ -605,13 +605,11 @@ void launch_img_coil2ext(const Plan& p, const float2* X, float2* ext, int batch,
                          hipStream_t s);
 // CGNR (reference E^H) kernels
 // step 1 / 2: also take the CGNR scalar step that reads this dot product (alpha / beta)
-void launch_cnr_dot_samples(const Plan& p, const float2* v, double* out_slot, hipStream_t s, int step = -1);
-void launch_cnr_dot_image(const Plan& p, const float2* v, bool masked, double* out_slot,
-                          hipStream_t s, int step = -1);
-void launch_cnr_scalars(const Plan& p, int step, double eps, hipStream_t s);
-void launch_cnr_update_image(const Plan& p, float2* fhat, float2* phat, const float2* z,
-                             int step, hipStream_t s);
-void launch_cnr_update_samples_dot(const Plan& p, const float2* rin, float2* r, const float2* v, hipStream_t s);
+void launch_cnr_dot(const Plan& p, const float2* v, int image, int slot, int step, double eps, const int* fl,
+                    hipStream_t s);
+void launch_cnr_update(const Plan& p, float2* fhat, const float2* phat, bool first, const float2* rin, float2* r,
+                       const float2* v, bool last, double eps, const int* fl, hipStream_t s);
+void launch_cnr_update_p(const Plan& p, float2* phat, const float2* z, const int* fl, hipStream_t s);
 void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 void launch_toep_layout(const float2* Khat, float* That, int64_t cells, int nl, int F, float scale,
                         hipStream_t s);

@@ -889,20 +889,67 @@ __global__ void __launch_bounds__(256) k_cnr_partials(const float2* v, const flo
   }
 }
 
-// r -= alpha v over the frame's samples, fused with the next dot_r partials:
-// the rows, lanes and summation order of k_cnr_partials over the updated r
-// (same block partials), so the pass over r is read once
+// The two updates that follow alpha, in one launch (on small plans a launch of its
+// own costs more than the 2 us either update takes; with the scalar steps taken in
+// k_cnr_reduce, p = z written by the transform itself and the last step ending at
+// f_hat, three steps are 37 launches instead of 58: 256^2 x 32 coils 1061 -> 869 us,
+// 128^2 x 8 coils CGLS(4) 1640 -> 1333 us).  Blocks below nsb:
+// r -= alpha v over the frame's samples, fused with the next dot_r partials: the
+// rows, lanes and summation order of k_cnr_partials over the updated r (same block
+// partials), so the pass over r is read once.  The others: f_hat += alpha w_hat p;
+// `first`: f_hat is written, not read (it starts at zero).
+struct CnrUpdate {
+  const float2* rin;
+  float2* r;
+  const float2* v;
+  const float* w;
+  const int64_t* foff;
+  const double* cnr;
+  double* partials;
+  const int* fmask;
+  float2* fhat;
+  const float2* phat;
+  int64_t Ntot;
+  int F, C, nsb, first, mask_nh, d, N0, N1;
+};
 template <int CP>
-__global__ void __launch_bounds__(256) k_cnr_update_samples_dot(const float2* rin, float2* r, const float2* v,
-                                                                const float* w, const int64_t* foff,
-                                                                const double* cnr, int F, int C, double* partials,
-                                                                const int* fmask) {
-  const int f = blockIdx.y;
-  if (fmask && fmask[f]) return;
+__global__ void __launch_bounds__(256) k_cnr_update(CnrUpdate a) {
+  const int f = blockIdx.y, C = a.C;
+  if (a.fmask && a.fmask[f]) return;
   constexpr int RPB = 256 / CP, U = 8;
   const int g = threadIdx.x / CP, cl = threadIdx.x % CP;
+  if ((int)blockIdx.x >= a.nsb) {
+    const int64_t stride = (int64_t)(gridDim.x - a.nsb) * RPB;
+    for (int c0 = 0; c0 < C; c0 += CP) {
+      const int c = c0 + cl;
+      if (c >= C) continue;
+      const float al = (float)a.cnr[(int64_t)3 * a.F * C + (int64_t)f * C + c];
+      float2* fh = a.fhat + (int64_t)f * a.Ntot * C + c;
+      const float2* ph = a.phat + (int64_t)f * a.Ntot * C + c;
+      for (int64_t i = (int64_t)(blockIdx.x - a.nsb) * RPB + g; i < a.Ntot; i += stride) {
+        const bool in = damp_in((uint32_t)i, a.N0, a.N1, a.d, a.mask_nh);
+        if (!in && !a.first) continue;
+        float2 ff = a.first ? make_float2(0.f, 0.f) : fh[i * C];
+        if (in) {
+          const float2 pp = ph[i * C];
+          ff.x += al * pp.x;
+          ff.y += al * pp.y;
+        }
+        fh[i * C] = ff;
+      }
+    }
+    return;
+  }
+  const float2* rin = a.rin;
+  float2* r = a.r;
+  const float2* v = a.v;
+  const float* w = a.w;
+  const int64_t* foff = a.foff;
+  const double* cnr = a.cnr;
+  double* partials = a.partials;
+  const int F = a.F, nsb = a.nsb;
   const int64_t r0 = foff[f], r1 = foff[f + 1];
-  const int64_t stride = (int64_t)gridDim.x * RPB;
+  const int64_t stride = (int64_t)nsb * RPB;
   __shared__ double sh[256];
   for (int c0 = 0; c0 < C; c0 += CP) {
     const int c = c0 + cl;
@@ -942,7 +989,7 @@ __global__ void __launch_bounds__(256) k_cnr_update_samples_dot(const float2* ri
     if (threadIdx.x < CP) {
       double t = 0.0;
       for (int k = 0; k < RPB; ++k) t += sh[k * CP + threadIdx.x];
-      if (c0 + threadIdx.x < C) partials[((int64_t)f * gridDim.x + blockIdx.x) * C + c0 + threadIdx.x] = t;
+      if (c0 + threadIdx.x < C) partials[((int64_t)f * nsb + blockIdx.x) * C + c0 + threadIdx.x] = t;
     }
     __syncthreads();
   }
@@ -951,10 +998,11 @@ __global__ void __launch_bounds__(256) k_cnr_update_samples_dot(const float2* ri
 // one block per frame: thread (coil cl, chunk j) sums partials b = j, j + 8, ...
 // in order, then chunk sums j = 0..7 are added in order (a fixed order: the
 // result does not depend on timing)
-// step 1 / 2 (else -1): the scalar step that reads this sum, taken here for the
-// same (frame, coil) -- alpha after dot_v, beta after the new dot_z (as k_cnr_scalars)
+// step: the scalar step that reads this sum, taken here for the same (frame, coil):
+// 0 after dot_r: stop where it is below eps (NFFTTraits.hpp:131); 3 the same after
+// the first dot_r; 1 alpha after dot_v; 2 beta after the new dot_z; -1 none
 __global__ void __launch_bounds__(256) k_cnr_reduce(const double* partials, int nb, int C, int F, double* cnr,
-                                                    int slot, const int* fmask, int step) {
+                                                    int slot, const int* fmask, int step, double eps) {
   constexpr int CB = 32, NJ = 256 / CB;
   __shared__ double sh[256];
   const int f = blockIdx.x;
@@ -975,7 +1023,12 @@ __global__ void __launch_bounds__(256) k_cnr_reduce(const double* partials, int 
       for (int jj = 0; jj < NJ; ++jj) u += sh[jj * CB + cl];
       const int64_t FC = (int64_t)F * C, idx = (int64_t)f * C + c;
       cnr[slot * FC + idx] = u;
-      if (step == 1) {          // alpha = dot_z / dot_v (u = dot_v)
+      if (step == 0) {
+        if (!(u >= eps)) cnr[5 * FC + idx] = 0.0;
+      } else if (step == 3) {
+        cnr[5 * FC + idx] = u >= eps ? 1.0 : 0.0;
+        cnr[3 * FC + idx] = cnr[4 * FC + idx] = 0.0;
+      } else if (step == 1) {   // alpha = dot_z / dot_v (u = dot_v)
         cnr[3 * FC + idx] = (cnr[5 * FC + idx] != 0.0) ? cnr[1 * FC + idx] / u : 0.0;
       } else if (step == 2) {   // beta = new dot_z / dot_z; dot_z = new (u = new dot_z)
         if (cnr[5 * FC + idx] != 0.0) {
@@ -988,71 +1041,32 @@ __global__ void __launch_bounds__(256) k_cnr_reduce(const double* partials, int 
   }
 }
 
-static void cnr_dot(const Plan& p, const float2* v, int image, double* dst_cnr, int slot, int step, hipStream_t s) {
+static void cnr_reduce(const Plan& p, int slot, const int* fl, int step, double eps, hipStream_t s) {
+  hipLaunchKernelGGL(k_cnr_reduce, dim3((unsigned)p.F), dim3(256), 0, s, p.partials, kCnrBlocks, p.C, p.F, p.cnr,
+                     slot, fl, step, eps);
+}
+
+// weighted squared norm per (frame, coil) of samples (image = 0) or damped images
+// (image = 1) into slot, then the scalar step (k_cnr_reduce)
+void launch_cnr_dot(const Plan& p, const float2* v, int image, int slot, int step, double eps, const int* fl,
+                    hipStream_t s) {
   const dim3 g(kCnrBlocks, p.F);
   const int nh = (int)(0.5 * p.N[0]);
-  if (p.C <= 8)
-    hipLaunchKernelGGL(k_cnr_partials<8>, g, dim3(256), 0, s, v, p.w, p.d_foff, p.Ntot, nh, p.d, p.N[0], p.N[1], p.C, image, p.partials, p.fmask);
-  else if (p.C <= 16)
-    hipLaunchKernelGGL(k_cnr_partials<16>, g, dim3(256), 0, s, v, p.w, p.d_foff, p.Ntot, nh, p.d, p.N[0], p.N[1], p.C, image, p.partials, p.fmask);
-  else
-    hipLaunchKernelGGL(k_cnr_partials<32>, g, dim3(256), 0, s, v, p.w, p.d_foff, p.Ntot, nh, p.d, p.N[0], p.N[1], p.C, image, p.partials, p.fmask);
-  hipLaunchKernelGGL(k_cnr_reduce, dim3((unsigned)p.F), dim3(256), 0, s, p.partials, kCnrBlocks, p.C, p.F, dst_cnr,
-                     slot, p.fmask, step);
+#define CGS_CNR(CP)                                                                                               \
+  hipLaunchKernelGGL(k_cnr_partials<CP>, g, dim3(256), 0, s, v, p.w, p.d_foff, p.Ntot, nh, p.d, p.N[0], p.N[1], \
+                     p.C, image, p.partials, fl)
+  if (p.C <= 8) CGS_CNR(8);
+  else if (p.C <= 16) CGS_CNR(16);
+  else CGS_CNR(32);
+#undef CGS_CNR
+  cnr_reduce(p, slot, fl, step, eps, s);
 }
 
-void launch_cnr_dot_samples(const Plan& p, const float2* v, double* cnr_slot_base, hipStream_t s, int step) {
-  // cnr_slot_base encodes the slot: pointer p.cnr + slot*F*C
-  const int slot = (int)((cnr_slot_base - p.cnr) / (p.F * p.C));
-  cnr_dot(p, v, 0, p.cnr, slot, step, s);
-}
-void launch_cnr_dot_image(const Plan& p, const float2* v, bool masked, double* cnr_slot_base, hipStream_t s,
-                          int step) {
-  (void)masked;
-  const int slot = (int)((cnr_slot_base - p.cnr) / (p.F * p.C));
-  cnr_dot(p, v, 1, p.cnr, slot, step, s);
-}
-
-// step 0: active &= dot_r >= eps (NFFTTraits.hpp:131); step 1: alpha; step 2: beta,
-// step 3: initialise (active = 1).
-__global__ void k_cnr_scalars(double* cnr, int FC, int step, double eps, const int* fmask, int C) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= FC) return;
-  if (fmask && fmask[idx / C]) return;
-  double* dot_r = cnr + 0 * FC;
-  double* dot_z = cnr + 1 * FC;
-  double* dot_v = cnr + 2 * FC;
-  double* alpha = cnr + 3 * FC;
-  double* beta = cnr + 4 * FC;
-  double* active = cnr + 5 * FC;
-  double* nv = cnr + 6 * FC;
-  if (step == 3) {
-    active[idx] = 1.0;
-    alpha[idx] = 0.0;
-    beta[idx] = 0.0;
-  } else if (step == 0) {
-    if (!(dot_r[idx] >= eps)) active[idx] = 0.0;
-  } else if (step == 1) {
-    alpha[idx] = (active[idx] != 0.0) ? dot_z[idx] / dot_v[idx] : 0.0;
-  } else {
-    if (active[idx] != 0.0) {
-      beta[idx] = nv[idx] / dot_z[idx];
-      dot_z[idx] = nv[idx];
-    }
-  }
-}
-
-void launch_cnr_scalars(const Plan& p, int step, double eps, hipStream_t s) {
-  const int n = p.F * p.C;
-  hipLaunchKernelGGL(k_cnr_scalars, dim3((n + 255) / 256), dim3(256), 0, s, p.cnr, n, step, eps, p.fmask, p.C);
-}
-
-// step 0: f_hat += alpha w_hat p_hat ; step 1: p_hat = active ? beta p_hat + z : p_hat.
+// p = beta p + z where the coil is active.
 // Blocks (pixel range, frame), lanes (pixel, coil): no index division per element.
 template <int CP>
-__global__ void __launch_bounds__(256) k_cnr_update_image(float2* fhat, float2* phat, const float2* z,
-                                                          const double* cnr, int F, int C, int64_t Ntot, int mask_nh,
-                                                          int d, int N0, int N1, int step, const int* fmask) {
+__global__ void __launch_bounds__(256) k_cnr_update_p(float2* phat, const float2* z, const double* cnr, int F, int C,
+                                                      int64_t Ntot, const int* fmask) {
   const int f = blockIdx.y;
   if (fmask && fmask[f]) return;
   constexpr int RPB = 256 / CP;
@@ -1063,61 +1077,47 @@ __global__ void __launch_bounds__(256) k_cnr_update_image(float2* fhat, float2* 
     const int c = c0 + cl;
     if (c >= C) continue;
     const int64_t fc = (int64_t)f * C + c;
-    float2* fh = fhat + (int64_t)f * Ntot * C + c;
+    if (cnr[5 * FC + fc] == 0.0) continue;
+    const float be = (float)cnr[4 * FC + fc];
     float2* ph = phat + (int64_t)f * Ntot * C + c;
-    if (step == 0) {
-      const float al = (float)cnr[3 * FC + fc];
-      for (int64_t i = (int64_t)blockIdx.x * RPB + g; i < Ntot; i += stride) {
-        if (!damp_in((uint32_t)i, N0, N1, d, mask_nh)) continue;
-        const float2 pp = ph[i * C];
-        float2 ff = fh[i * C];
-        ff.x += al * pp.x;
-        ff.y += al * pp.y;
-        fh[i * C] = ff;
-      }
-    } else {
-      if (cnr[5 * FC + fc] == 0.0) continue;
-      const float be = (float)cnr[4 * FC + fc];
-      const float2* zz = z + (int64_t)f * Ntot * C + c;
-      for (int64_t i = (int64_t)blockIdx.x * RPB + g; i < Ntot; i += stride) {
-        const float2 zv = zz[i * C];
-        float2 pp = ph[i * C];
-        pp.x = be * pp.x + zv.x;
-        pp.y = be * pp.y + zv.y;
-        ph[i * C] = pp;
-      }
+    const float2* zz = z + (int64_t)f * Ntot * C + c;
+    for (int64_t i = (int64_t)blockIdx.x * RPB + g; i < Ntot; i += stride) {
+      const float2 zv = zz[i * C];
+      float2 pp = ph[i * C];
+      pp.x = be * pp.x + zv.x;
+      pp.y = be * pp.y + zv.y;
+      ph[i * C] = pp;
     }
   }
 }
 
-void launch_cnr_update_image(const Plan& p, float2* fhat, float2* phat, const float2* z, int step, hipStream_t s) {
-  const dim3 g((unsigned)std::max(64, 2048 / std::max(1, p.F)), (unsigned)p.F);
-  const int nh = (int)(0.5 * p.N[0]);
-  if (p.C <= 8)
-    hipLaunchKernelGGL(k_cnr_update_image<8>, g, dim3(256), 0, s, fhat, phat, z, p.cnr, p.F, p.C, p.Ntot, nh, p.d,
-                       p.N[0], p.N[1], step, p.fmask);
-  else if (p.C <= 16)
-    hipLaunchKernelGGL(k_cnr_update_image<16>, g, dim3(256), 0, s, fhat, phat, z, p.cnr, p.F, p.C, p.Ntot, nh, p.d,
-                       p.N[0], p.N[1], step, p.fmask);
-  else
-    hipLaunchKernelGGL(k_cnr_update_image<32>, g, dim3(256), 0, s, fhat, phat, z, p.cnr, p.F, p.C, p.Ntot, nh, p.d,
-                       p.N[0], p.N[1], step, p.fmask);
+static unsigned cnr_image_blocks(const Plan& p) { return (unsigned)std::max(64, 2048 / std::max(1, p.F)); }
+
+void launch_cnr_update_p(const Plan& p, float2* phat, const float2* z, const int* fl, hipStream_t s) {
+  const dim3 g(cnr_image_blocks(p), (unsigned)p.F);
+#define CGS_CNR(CP) hipLaunchKernelGGL(k_cnr_update_p<CP>, g, dim3(256), 0, s, phat, z, p.cnr, p.F, p.C, p.Ntot, fl)
+  if (p.C <= 8) CGS_CNR(8);
+  else if (p.C <= 16) CGS_CNR(16);
+  else CGS_CNR(32);
+#undef CGS_CNR
 }
 
-// r = rin - alpha v (rin == r: in place), then dot_r (slot 0) from the fused pass's partials
-void launch_cnr_update_samples_dot(const Plan& p, const float2* rin, float2* r, const float2* v, hipStream_t s) {
-  const dim3 g(kCnrBlocks, p.F);
-  if (p.C <= 8)
-    hipLaunchKernelGGL(k_cnr_update_samples_dot<8>, g, dim3(256), 0, s, rin, r, v, p.w, p.d_foff, p.cnr, p.F, p.C,
-                       p.partials, p.fmask);
-  else if (p.C <= 16)
-    hipLaunchKernelGGL(k_cnr_update_samples_dot<16>, g, dim3(256), 0, s, rin, r, v, p.w, p.d_foff, p.cnr, p.F, p.C,
-                       p.partials, p.fmask);
-  else
-    hipLaunchKernelGGL(k_cnr_update_samples_dot<32>, g, dim3(256), 0, s, rin, r, v, p.w, p.d_foff, p.cnr, p.F, p.C,
-                       p.partials, p.fmask);
-  hipLaunchKernelGGL(k_cnr_reduce, dim3((unsigned)p.F), dim3(256), 0, s, p.partials, kCnrBlocks, p.C, p.F, p.cnr, 0,
-                     p.fmask, -1);
+// f_hat += alpha w_hat p (first: from zero); unless `last`, r = rin - alpha v (rin
+// may be r) and dot_r (slot 0) with its stop test
+void launch_cnr_update(const Plan& p, float2* fhat, const float2* phat, bool first, const float2* rin, float2* r,
+                       const float2* v, bool last, double eps, const int* fl, hipStream_t s) {
+  CnrUpdate a{};
+  a.rin = rin; a.r = r; a.v = v; a.w = p.w; a.foff = p.d_foff; a.cnr = p.cnr; a.partials = p.partials;
+  a.fmask = fl; a.fhat = fhat; a.phat = phat; a.Ntot = p.Ntot; a.F = p.F; a.C = p.C;
+  a.nsb = last ? 0 : kCnrBlocks;
+  a.first = first ? 1 : 0;
+  a.mask_nh = (int)(0.5 * p.N[0]);
+  a.d = p.d; a.N0 = p.N[0]; a.N1 = p.N[1];
+  const dim3 g((unsigned)a.nsb + cnr_image_blocks(p), (unsigned)p.F);
+  if (p.C <= 8) hipLaunchKernelGGL(k_cnr_update<8>, g, dim3(256), 0, s, a);
+  else if (p.C <= 16) hipLaunchKernelGGL(k_cnr_update<16>, g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_cnr_update<32>, g, dim3(256), 0, s, a);
+  if (!last) cnr_reduce(p, 0, fl, 0, eps, s);
 }
 
 // Toeplitz spectrum: grid order Khat[f][r + cells*pos] -> conv-pass layout

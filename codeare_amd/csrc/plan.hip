@@ -521,59 +521,58 @@ static int op_EH_true(Plan& p, const float2* y, float2* x, const float2* pv, flo
 // Default: the plan's NFFT (gridding + adjoint FFT passes, masked forward FFT
 // passes + gather); the off-resonance model supplies its own.
 struct CnrOps {
-  std::function<int(const float2* r)> adj_w;
+  std::function<int(const float2* r, float2* X)> adj_w;
   std::function<int(const float2* x, float2* v)> fwd_masked;
 };
 
 // NFFT3 weighted damped CGNR (NFFTTraits.hpp:122-138) for every (frame, coil):
-// f_hat = ITrafo(y), written to p.Xc2.  Frames flagged in fl are skipped.
+// f_hat = ITrafo(y), written to p.Xc2.  Frames flagged in fl are skipped.  A step's
+// new residual, its adjoint z and the next direction serve the next step, so the
+// last step ends with f_hat: nothing reads the others.
 static int cgnr(Plan& p, const float2* y, int maxit, double eps, const int* fl, const CnrOps* ops = nullptr) {
-  const size_t Fb = sizeof(int) * p.F;
-  if (fl && fl != p.fmask) HIPCHK(hipMemcpyAsync(p.fmask, fl, Fb, hipMemcpyDeviceToDevice, p.stream));
-  if (!fl) launch_fill_int(p.fmask, 0, p.F, p.stream);
-  const int* m = p.fmask;
   const size_t ybytes = sizeof(float2) * (size_t)p.Mtot * p.C;
   const size_t xbytes = sizeof(float2) * (size_t)p.F * p.Ntot * p.C;
-  const int FC = p.F * p.C;
   float2* r = p.ybuf[2];
   float2* v = p.ybuf[3];
+  if (maxit <= 0) {
+    launch_zero(p.Xc2, xbytes, p.stream);
+    return CGS_OK;
+  }
   {
     // r = y - A 0 = y: the first step reads y and writes r, so y is not copied
     Prof pr(p, CGS_K_CG, 1.0 * ybytes);
-    launch_cnr_scalars(p, 3, eps, p.stream);
-    launch_cnr_dot_samples(p, y, p.cnr + 0 * FC, p.stream);                    // dot_r
+    launch_cnr_dot(p, y, 0, 0, 3, eps, fl, p.stream);                          // dot_r; dot_r < eps -> stop
   }
-  auto adj_w = [&](const float2* rr) -> int {                                   // z = A^H W r
-    if (ops) return ops->adj_w(rr);
-    CHK(gridding(p, rr, true, m));
-    return fft_adjoint(p, p.Xc, m);
+  auto adj_w = [&](const float2* rr, float2* X) -> int {                        // z = A^H W r
+    if (ops) return ops->adj_w(rr, X);
+    CHK(gridding(p, rr, true, fl));
+    return fft_adjoint(p, X, fl);
   };
   auto fwd_masked = [&](const float2* xx, float2* vv) -> int {                 // v = A(w_hat p)
     if (ops) return ops->fwd_masked(xx, vv);
-    CHK(fft_forward(p, 3, xx, m));
-    return interp(p, vv, m);
+    CHK(fft_forward(p, 3, xx, fl));
+    return interp(p, vv, fl);
   };
-  CHK(adj_w(y));
+  CHK(adj_w(y, p.Xc3));                                                         // p = z
   {
-    Prof pr(p, CGS_K_CG, 3.0 * xbytes);
-    launch_cnr_dot_image(p, p.Xc, true, p.cnr + 1 * FC, p.stream);             // dot_z
-    HIPCHK(hipMemcpyAsync(p.Xc3, p.Xc, xbytes, hipMemcpyDeviceToDevice, p.stream));   // p = z
-    launch_zero(p.Xc2, xbytes, p.stream);                                       // f_hat = 0
+    Prof pr(p, CGS_K_CG, 1.0 * xbytes);
+    launch_cnr_dot(p, p.Xc3, 1, 1, -1, eps, fl, p.stream);                     // dot_z
   }
   for (int l = 0; l < maxit; ++l) {
-    launch_cnr_scalars(p, 0, eps, p.stream);                                   // dot_r < eps -> stop
+    const bool last = l + 1 == maxit;
     CHK(fwd_masked(p.Xc3, v));                                                  // v = A(w_hat p)
     {
-      Prof pr(p, CGS_K_CG, 4.0 * xbytes + 4.0 * ybytes);
-      launch_cnr_dot_samples(p, v, p.cnr + 2 * FC, p.stream, 1);               // dot_v; alpha
-      launch_cnr_update_image(p, p.Xc2, p.Xc3, nullptr, 0, p.stream);          // f_hat += a w_hat p
-      launch_cnr_update_samples_dot(p, l == 0 ? y : r, r, v, p.stream);        // r -= a v; dot_r
+      Prof pr(p, CGS_K_CG, (l ? 3.0 : 2.0) * xbytes + (last ? 1.0 : 4.0) * ybytes);
+      launch_cnr_dot(p, v, 0, 2, 1, eps, fl, p.stream);                        // dot_v; alpha
+      // f_hat += a w_hat p; r -= a v; dot_r; dot_r < eps -> stop
+      launch_cnr_update(p, p.Xc2, p.Xc3, l == 0, l == 0 ? y : r, r, v, last, eps, fl, p.stream);
     }
-    CHK(adj_w(r));                                                              // z = A^H W r
+    if (last) break;
+    CHK(adj_w(r, p.Xc));                                                        // z = A^H W r
     {
       Prof pr(p, CGS_K_CG, 4.0 * xbytes);
-      launch_cnr_dot_image(p, p.Xc, true, p.cnr + 6 * FC, p.stream, 2);        // dot_z (new); beta
-      launch_cnr_update_image(p, nullptr, p.Xc3, p.Xc, 1, p.stream);           // p = b p + z
+      launch_cnr_dot(p, p.Xc, 1, 6, 2, eps, fl, p.stream);                     // dot_z (new); beta
+      launch_cnr_update_p(p, p.Xc3, p.Xc, fl, p.stream);                       // p = b p + z
     }
   }
   return CGS_OK;
@@ -2681,7 +2680,7 @@ int cgs_nfft_inverse_ref(cgs_plan plan, int frame, const void* f, void* img, int
     Plan& q = *p.b0q;
     launch_y_ext2int(q, fd, p.ybuf[0], batch, frame, p.stream);
     CnrOps ops;
-    ops.adj_w = [&](const float2* r) { return b0_adjoint(p, r, true, p.Xc); };
+    ops.adj_w = [&](const float2* r, float2* X) { return b0_adjoint(p, r, true, X); };
     ops.fwd_masked = [&](const float2* x, float2* v) { return b0_forward(p, x, v, true); };
     float* w_keep = p.w;
     int* sframe_keep = p.sframe;
