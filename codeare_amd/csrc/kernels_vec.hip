@@ -995,16 +995,19 @@ __global__ void __launch_bounds__(256) k_cnr_update(CnrUpdate a) {
   }
 }
 
-// one block per frame: thread (coil cl, chunk j) sums partials b = j, j + 8, ...
-// in order, then chunk sums j = 0..7 are added in order (a fixed order: the
-// result does not depend on timing)
+// one block of 32 CB threads per frame: thread (coil cl, chunk j) sums partials
+// b = j, j + 32, ... in order, then chunk sums j = 0..31 are added in order (a fixed
+// order: the result does not depend on timing).  32 chunks, so that a thread's eight
+// loads are one round trip (8 chunks, four dependent rounds of loads: 3.3 us a launch
+// at 8 coils, of which 1.3 are the launch; so: 2.3 us).
 // step: the scalar step that reads this sum, taken here for the same (frame, coil):
 // 0 after dot_r: stop where it is below eps (NFFTTraits.hpp:131); 3 the same after
 // the first dot_r; 1 alpha after dot_v; 2 beta after the new dot_z; -1 none
-__global__ void __launch_bounds__(256) k_cnr_reduce(const double* partials, int nb, int C, int F, double* cnr,
-                                                    int slot, const int* fmask, int step, double eps) {
-  constexpr int CB = 32, NJ = 256 / CB;
-  __shared__ double sh[256];
+template <int CB>
+__global__ void __launch_bounds__(32 * CB) k_cnr_reduce(const double* partials, int nb, int C, int F, double* cnr,
+                                                        int slot, const int* fmask, int step, double eps) {
+  constexpr int NJ = 32;
+  __shared__ double sh[NJ * CB];
   const int f = blockIdx.x;
   if (fmask && fmask[f]) return;
   const int cl = threadIdx.x % CB, j = threadIdx.x / CB;
@@ -1042,8 +1045,14 @@ __global__ void __launch_bounds__(256) k_cnr_reduce(const double* partials, int 
 }
 
 static void cnr_reduce(const Plan& p, int slot, const int* fl, int step, double eps, hipStream_t s) {
-  hipLaunchKernelGGL(k_cnr_reduce, dim3((unsigned)p.F), dim3(256), 0, s, p.partials, kCnrBlocks, p.C, p.F, p.cnr,
-                     slot, fl, step, eps);
+  const dim3 g((unsigned)p.F);
+#define CGS_CNR(CB)                                                                                              \
+  hipLaunchKernelGGL(k_cnr_reduce<CB>, g, dim3(32 * CB), 0, s, p.partials, kCnrBlocks, p.C, p.F, p.cnr, slot, fl, \
+                     step, eps)
+  if (p.C <= 8) CGS_CNR(8);
+  else if (p.C <= 16) CGS_CNR(16);
+  else CGS_CNR(32);
+#undef CGS_CNR
 }
 
 // weighted squared norm per (frame, coil) of samples (image = 0) or damped images
