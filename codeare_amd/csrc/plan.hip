@@ -255,17 +255,34 @@ static bool fft_reg_enabled() {
   return on;
 }
 
+// Axis-0 passes of one or two coils with few rows, which stay on k_fft: a block of
+// k_fft_pt takes 16 (8) rows there, so few rows are few blocks, and each of their
+// accesses is scattered over its rows, while k_fft gives every row a block and is slower
+// only once its blocks are more than fit the chip at a time.  First pass of E and last of
+// E^H W together, k_fft_pt / k_fft in us.  One coil: 144 points 11.1 / 12.7 (72 rows), 192
+// points 14.4 / 11.9 (192), 256 points 16.6 / 12.3 (256), 17.5 / 14.1 (1024), 384 points
+// 21.7 / 14.8 (384), 22.7 / 24.8 (1152), 512 points 24.4 / 13.5 (256), 26.4 / 17.9 (1024);
+// 243 points level.  Two coils: 256 points 13.2 / 12.6 (128), and first and last Toeplitz
+// pass 15.9 / 13.4; 384 points 17.8 / 15.9 (192), 20.2 / 20.8 (768), 512 points 20.3 / 14.9
+// (256), 21.6 / 19.5 (768), 20.8 / 22.0 (1024); 192, 288 to 324 and 432 to 486 points are
+// level or k_fft_pt's.  Three coils: k_fft_pt from 64 points on.
+static bool fft_few_rows(const FftArgs& a) {
+  if (a.inner > 2 || a.n > 512) return false;   // (above 512 points k_fft takes 2 to 9 times as long)
+  if (a.inner == 1) return a.n >= 192 && a.n % 2 == 0 && a.outers <= 1024;
+  return a.n >= 256 && a.n % 128 == 0 && 2 * a.outers <= 3 * a.n;
+}
+
 static void fft_finish(FftArgs& a) {
   // k_fft_r8 at 256, 384 and 512 points (why: kernels_fft_reg.hip), k_fft_pt at its
-  // lengths, the LDS kernel k_fft at the others: every stage of k_fft passes
-  // the line through LDS, which costs 2 to 9 times the memory traffic's time
+  // lengths except on few rows (above), the LDS kernel k_fft elsewhere: every stage of
+  // k_fft passes the line through LDS, which costs 2 to 9 times the memory traffic's time
   // (432-point lines, 12 coils: 22.4 us a pass against 8.8; the Toeplitz
   // convolution at 576 points, 20 coils: 508 against 31 us)
   const bool reg = fft_reg_enabled();
   a.lines_log2 = 0;
   while ((1 << a.lines_log2) < a.inner && a.lines_log2 < 4) ++a.lines_log2;
   a.use_reg = reg && fft_reg_supported(a);
-  a.use_pt = reg && !a.use_reg && fft_pt_supported(a);
+  a.use_pt = reg && !a.use_reg && fft_pt_supported(a) && !fft_few_rows(a);
   a.lb = (a.use_reg || a.use_pt) ? 16 : pick_lb(a.inner, a.n);
   a.lb_log2 = 0;
   while ((1 << a.lb_log2) < a.lb) ++a.lb_log2;
