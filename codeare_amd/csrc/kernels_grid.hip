@@ -13,6 +13,7 @@
 // a fixed summation order (deterministic).  Tiles whose visit lists are long
 // (the k-space centre of radial trajectories) are split across several items
 // that write partial tiles, summed afterwards in a fixed order.
+#include <algorithm>
 #include <cstdlib>
 
 #include "cgs_internal.hpp"
@@ -916,6 +917,17 @@ void launch_grid_reg(const GridArgs& a, const int4* vrec, int cgr, int nitems, i
   else grid_reg_taps<32>(a, vrec, nitems, g, shm, s);
 }
 
+// Launches over n items x groups in one grid dimension, `threads` a block: that dimension
+// holds fewer than 2^32 threads, which long series of volumes with many coils exceed (the
+// 3D gather of 38 frames of 128^3 x 16 coils has 4.2 M blocks of 1024 threads), so they
+// go in several launches.  go(first item, items); items start at multiples of `step`.
+template <class Go>
+static void launch_slices(int n, int groups, int threads, int step, Go&& go) {
+  const int64_t most = (int64_t)(0xffffffffu / (unsigned)threads) / groups / step * step;
+  const int64_t per = std::max<int64_t>(step, most);
+  for (int64_t i = 0; i < n; i += per) go(i, (int)std::min<int64_t>(per, n - i));
+}
+
 // ---------------------------------------------------------------------------
 // adjoint B^T on the matrix cores (2D, 8x8 tiles).  The tile's grid values are
 // D[cell][col] (64 cells x the real columns re/im of a coil group) and the work
@@ -1162,7 +1174,7 @@ GmShape gm_shape(int C) { return C <= 8 ? GmShape{8, 1} : GmShape{4, (C + 15) / 
 
 template <int R, int NW>
 static void grid_mfma_taps(const GridArgs& a, const int4* vrec, int nblocks, int ng, hipStream_t s) {
-  const dim3 g((unsigned)nblocks * (unsigned)ng), b(64 * NW);
+  const dim3 g((unsigned)nblocks * (unsigned)ng), b(64 * NW);   // fewer than 2^32 threads: launch_slices
 #define CGS_GM(TP)                                                                                   \
   do {                                                                                               \
     if (a.C % 2 == 0) hipLaunchKernelGGL((k_grid_mfma<TP, R, NW, true>), g, b, 0, s, a, vrec, ng);    \
@@ -1181,8 +1193,12 @@ static void grid_mfma_taps(const GridArgs& a, const int4* vrec, int nblocks, int
 void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nblocks, hipStream_t s) {
   if (nblocks == 0) return;
   const GmShape sh = gm_shape(a.C);
-  if (sh.waves == 8) grid_mfma_taps<16, 8>(a, vrec, nblocks, sh.groups, s);
-  else grid_mfma_taps<32, 4>(a, vrec, nblocks, sh.groups, s);
+  launch_slices(nblocks, sh.groups, 64 * sh.waves, 1, [&](int64_t first, int n) {
+    GridArgs b = a;
+    b.gwaves = a.gwaves + first * sh.waves;
+    if (sh.waves == 8) grid_mfma_taps<16, 8>(b, vrec, n, sh.groups, s);
+    else grid_mfma_taps<32, 4>(b, vrec, n, sh.groups, s);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -1413,8 +1429,13 @@ static void grid_mfma3_taps(const GridArgs& a, const int4* vrec, int nitems, int
 
 void launch_grid_mfma3(const GridArgs& a, const int4* vrec, int nitems, hipStream_t s) {
   if (nitems == 0) return;
-  if (a.C <= 8) grid_mfma3_taps<16>(a, vrec, nitems, 1, s);
-  else grid_mfma3_taps<32>(a, vrec, nitems, (a.C + 15) / 16, s);
+  const int ng = a.C <= 8 ? 1 : (a.C + 15) / 16;
+  launch_slices(nitems, ng, 512, 1, [&](int64_t first, int n) {
+    GridArgs b = a;
+    b.items = a.items + first;
+    if (a.C <= 8) grid_mfma3_taps<16>(b, vrec, n, ng, s);
+    else grid_mfma3_taps<32>(b, vrec, n, ng, s);
+  });
 }
 
 size_t grid_atomic_lds(int d, int T, int taps, int CG, int rowstride) {
@@ -1841,22 +1862,26 @@ void launch_interp_cs3(const SampArgs& a, const int4* items, int nitems, int T, 
   const size_t E = (size_t)T + a.taps - 1;
   const size_t shm = sizeof(float2) * E * (E * E + (split ? ppad : 0)) * 2;
   const int ng = (a.C + 1) / 2;
-  const dim3 g((unsigned)((nitems + 7) / 8 * 8) * (unsigned)ng);
-#define CGS_IC3(NT_, SP_)                                                                                        \
-  do {                                                                                                         \
-    if (T == 8) hipLaunchKernelGGL((k_interp_cs3<8, NT_, 8, SP_>), g, dim3(NT_), shm, s, a, items, nitems, ng, T, nt0, nt1, ppad); \
-    else hipLaunchKernelGGL((k_interp_cs3<8, NT_, 0, SP_>), g, dim3(NT_), shm, s, a, items, nitems, ng, T, nt0, nt1, ppad);        \
+  const int nt = threads >= 1024 ? 1024 : threads >= 512 ? 512 : 256;
+  launch_slices(nitems, ng, nt, 8, [&](int64_t first, int n) {
+    const int4* it = items + first;
+    const dim3 g((unsigned)((n + 7) / 8 * 8) * (unsigned)ng);
+#define CGS_IC3(NT_, SP_)                                                                                         \
+  do {                                                                                                            \
+    if (T == 8) hipLaunchKernelGGL((k_interp_cs3<8, NT_, 8, SP_>), g, dim3(NT_), shm, s, a, it, n, ng, T, nt0, nt1, ppad); \
+    else hipLaunchKernelGGL((k_interp_cs3<8, NT_, 0, SP_>), g, dim3(NT_), shm, s, a, it, n, ng, T, nt0, nt1, ppad);        \
   } while (0)
-  if (split) {
-    if (threads >= 1024) CGS_IC3(1024, 1);
-    else if (threads >= 512) CGS_IC3(512, 1);
-    else CGS_IC3(256, 1);
-  } else {
-    if (threads >= 1024) CGS_IC3(1024, 0);
-    else if (threads >= 512) CGS_IC3(512, 0);
-    else CGS_IC3(256, 0);
-  }
+    if (split) {
+      if (nt == 1024) CGS_IC3(1024, 1);
+      else if (nt == 512) CGS_IC3(512, 1);
+      else CGS_IC3(256, 1);
+    } else {
+      if (nt == 1024) CGS_IC3(1024, 0);
+      else if (nt == 512) CGS_IC3(512, 0);
+      else CGS_IC3(256, 0);
+    }
 #undef CGS_IC3
+  });
 }
 
 void launch_interp_lds3(const SampArgs& a, const int4* items, int nitems, int T, int nt0, int nt1, int cg, int maxs,

@@ -113,3 +113,28 @@ def test_nan_in_one_frame(cgs, toeplitz):
     assert e0 <= (1e-5 if rep["iters"][0] == r0["iters"][0] else 1e-3)
     assert rep["iters"][1] <= 1
     assert np.all(np.isfinite(xs[..., 0]))
+
+
+def test_3d_gather_of_a_long_series(cgs):
+    """608 frames of 12^3 x 512 coils, one sample in each of a frame's 27 tiles: the 3D
+    gather's 16 416 items x 256 coil pairs are more threads than one grid dimension holds.
+    Every frame is the same problem as its own plan's, so the samples agree to rounding
+    (the same sums: 1e-6), those of the last frames among them."""
+    rng = np.random.default_rng(19)
+    N, C, F, n = (12, 12, 12), 512, 608, 18
+    t = np.array([3.5, -5.5, -1.5]) / n   # cells 3, 12 and 16: one in each of an axis' three tiles
+    k = np.asfortranarray(np.stack(np.meshgrid(t, t, t, indexing="ij")).reshape(3, -1).astype(np.float32))
+    M = k.shape[1]
+    S = rand_img(rng, N + (C,))
+    x = rand_img(rng, N + (4,))
+    one = cgs.Plan(N, M, 1.5, 3, ncoils=C)
+    P = cgs.Plan(N, M * F, 1.5, 3, ncoils=C, frame_offsets=np.arange(F + 1, dtype=np.int64) * M)
+    for p, reps in ((one, 1), (P, F)):
+        p.kspace(np.asfortranarray(np.tile(k, (1, reps))))
+        p.weights(np.ones(M * reps, np.float32))
+        p.sensitivities(S)
+    y = P.E(np.asfortranarray(np.tile(x, (1, 1, 1, F // 4)))).reshape(F, M * C)
+    for f in range(4):
+        y1 = one.E(np.asfortranarray(x[..., f])).reshape(-1, order="F")
+        worst = max(rel(y[g], y1) for g in (*range(f, F, 101 * 4), F - 4 + f))
+        assert worst <= 1e-6, (f, worst)
