@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "cgs_internal.hpp"
+#include "host_threads.hpp"
 
 struct cgs_plan_s {
   cgs::Plan p;
@@ -901,24 +902,20 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
   std::vector<int> hframe((size_t)M);
   {
     const int nthr = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    std::vector<std::thread> th;
-    for (int t = 0; t < nthr; ++t) {
-      th.emplace_back([&, t]() {
-        for (int64_t s = t; s < M; s += nthr) {
-          const int64_t j = perm[s];
-          hframe[s] = frame[j];
-          for (int a = 0; a < d; ++a) {
-            int b = cell[j * d + a] - m;
-            b %= p.n[a];
-            if (b < 0) b += p.n[a];
-            hbase[s * d + a] = b;
-            for (int q = 0; q < taps; ++q)
-              hpsi[(s * d + a) * taps + q] = (float)kb_phi(frac[j * d + a] + m - q, m, p.b[a]);
-          }
+    run_shares(nthr, [&](int t) {
+      for (int64_t s = t; s < M; s += nthr) {
+        const int64_t j = perm[s];
+        hframe[s] = frame[j];
+        for (int a = 0; a < d; ++a) {
+          int b = cell[j * d + a] - m;
+          b %= p.n[a];
+          if (b < 0) b += p.n[a];
+          hbase[s * d + a] = b;
+          for (int q = 0; q < taps; ++q)
+            hpsi[(s * d + a) * taps + q] = (float)kb_phi(frac[j * d + a] + m - q, m, p.b[a]);
         }
-      });
-    }
-    for (auto& x : th) x.join();
+      }
+    });
   }
   // interp items: runs of samples of one frame
   const int ipw = (d == 3) ? 4 : 16;
@@ -982,7 +979,7 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
   {
     // (a thread per 32768 visits: starting one costs about as much as that many records)
     const int nthr = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(16u, std::thread::hardware_concurrency()), nvis >> 15));
-    auto tiles = [&](int th) {
+    run_shares(nthr, [&](int th) {
       std::vector<int4> tmp;
       // thread th takes the tiles of its share of the visits
       const int64_t k0 = std::lower_bound(vcnt.begin(), vcnt.end() - 1, nvis * th / nthr) - vcnt.begin();
@@ -1014,24 +1011,17 @@ static int build_samples(Plan& p, const float* k, bool sweep = true) {
           rc.w = (d == 3) ? (int)(((uint32_t)rel[2] & 0xffffu) | ((uint32_t)lo[2] << 16) | ((uint32_t)hi[2] << 24)) : 0;
           vrec[v] = rc;
         }
-        if (vcnt[kk + 1] - vcnt[kk] > 1) {   // counting sort by rel1 in (-taps, T)
-          const int nc = T + taps;   // (tiles wider than 69 cells stay unsorted)
-          int64_t pos[80] = {0};
-          const int4* src = vrec.data() + vcnt[kk];
-          const int64_t n = vcnt[kk + 1] - vcnt[kk];
-          tmp.assign(src, src + n);
-          if (nc + 1 <= (int)(sizeof(pos) / sizeof(pos[0]))) {
-            for (const int4& r : tmp) pos[(r.y >> 16) + taps + 1]++;
-            for (int q = 0; q < nc; ++q) pos[q + 1] += pos[q];
-            for (const int4& r : tmp) vrec[vcnt[kk] + pos[(r.y >> 16) + taps]++] = r;
-          }
+        // counting sort by rel1 in (-taps, T) (tiles wider than 69 cells stay unsorted)
+        const int nc = T + taps;
+        int64_t pos[80] = {0};
+        if (vcnt[kk + 1] - vcnt[kk] > 1 && nc + 1 <= (int)(sizeof(pos) / sizeof(pos[0]))) {
+          tmp.assign(vrec.data() + vcnt[kk], vrec.data() + vcnt[kk + 1]);
+          for (const int4& r : tmp) pos[(r.y >> 16) + taps + 1]++;
+          for (int q = 0; q < nc; ++q) pos[q + 1] += pos[q];
+          for (const int4& r : tmp) vrec[vcnt[kk] + pos[(r.y >> 16) + taps]++] = r;
         }
       }
-    };
-    std::vector<std::thread> th;
-    for (int t = 1; t < nthr; ++t) th.emplace_back(tiles, t);
-    tiles(0);
-    for (auto& x : th) x.join();
+    });
   }
   std::vector<GridItem> gitems;
   std::vector<ReduceItem> ritems;
