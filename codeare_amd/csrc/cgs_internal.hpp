@@ -533,11 +533,11 @@ LaunchEvents& launch_events();
     }                                                                                           \
   } while (0)
 
-void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
+int launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
 bool fft_reg_supported(const FftArgs& a);
 bool fft_pt_supported(const FftArgs& a);
-void launch_fft_pt(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
-void launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
+bool launch_fft_pt(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
+bool launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s);
 bool toep_pad_crop_supported(int N0, int N1, int C);
 bool toep_conv_supported(int N0, int N1, int C);
 bool toep_half_supported(int N0, int N1, int C);

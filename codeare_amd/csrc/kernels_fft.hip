@@ -329,15 +329,8 @@ __global__ void __launch_bounds__(kFftThreads) k_fft(FftArgs a) {
 
 size_t fft_lds_bytes(const FftArgs& a) { return sizeof(float2) * ((size_t)a.lb * a.ldn + a.n); }
 
-void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
-  if (a.use_pt) {
-    launch_fft_pt(a, ld_mode, st_mode, s);
-    return;
-  }
-  if (a.use_reg) {
-    launch_fft_reg(a, ld_mode, st_mode, s);
-    return;
-  }
+// a pass on k_fft; false: no such kernel
+static bool launch_fft_lds(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   const int64_t nib = (a.inner + a.lb - 1) / a.lb;
   const dim3 grid((unsigned)(nib * a.outers));
   const size_t shm = fft_lds_bytes(a);
@@ -348,7 +341,7 @@ void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
       CGS_LAUNCH((k_fft<L, S_, 512, CV>), grid, dim3(kFftThreads), shm, s, a);           \
     else                                                                                 \
       CGS_LAUNCH((k_fft<L, S_, 4096, CV>), grid, dim3(kFftThreads), shm, s, a);          \
-    return;                                                                              \
+    return true;                                                                         \
   }
   CGS_FFT_CASE(0, 0, 0)
   CGS_FFT_CASE(1, 0, 0)
@@ -359,6 +352,20 @@ void launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   CGS_FFT_CASE(0, 0, 1)
   CGS_FFT_CASE(0, 2, 0)
 #undef CGS_FFT_CASE
+  return false;
+}
+
+// the kernels exist in the modes that the passes use; a pass in another one is an error
+// of its caller, not a launch left out
+int launch_fft(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
+  const bool ok = a.use_pt ? launch_fft_pt(a, ld_mode, st_mode, s)
+                  : a.use_reg ? launch_fft_reg(a, ld_mode, st_mode, s)
+                              : launch_fft_lds(a, ld_mode, st_mode, s);
+  if (ok) return CGS_OK;
+  set_error("no FFT kernel of " + std::to_string(a.n) + " points for load mode " + std::to_string(ld_mode) +
+            ", store mode " + std::to_string(st_mode) + (a.That ? ", convolution" : "") + ", sign " +
+            std::to_string(a.sign));
+  return CGS_ERR_UNSUPPORTED;
 }
 
 }  // namespace cgs

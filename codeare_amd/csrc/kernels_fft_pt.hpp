@@ -312,14 +312,14 @@ __global__ void __launch_bounds__(16 * T) k_fft_pt(FftArgs a) {
 }  // namespace
 
 template <int P, int T>
-static void launch_pt(const FftArgs& a, int ld, int st, hipStream_t s) {
+static bool launch_pt(const FftArgs& a, int ld, int st, hipStream_t s) {   // false: no such kernel
   const int R = 16 >> a.lines_log2;
   const dim3 grid((unsigned)((a.outers + R - 1) / R * ((a.inner + 15) / 16)));
   const int conv = a.That != nullptr;
 #define CGS_PT_CASE(L, S_, CV, SG_)                                                                  \
   if (ld == L && st == S_ && conv == CV && a.sign == SG_) {                                          \
     CGS_LAUNCH((k_fft_pt<P, T, L, S_, CV, SG_>), grid, dim3(16 * T), 0, s, a);                        \
-    return;                                                                                          \
+    return true;                                                                                        \
   }
   CGS_PT_CASE(0, 0, 0, -1)
   CGS_PT_CASE(0, 0, 0, 1)
@@ -331,6 +331,7 @@ static void launch_pt(const FftArgs& a, int ld, int st, hipStream_t s) {
   CGS_PT_CASE(0, 0, 1, -1)
   CGS_PT_CASE(0, 2, 0, 1)
 #undef CGS_PT_CASE
+  return false;
 }
 
 }  // namespace cgs

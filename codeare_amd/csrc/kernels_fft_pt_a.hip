@@ -27,22 +27,22 @@ bool fft_pt_supported(const FftArgs& a) {
   return maps < lim && R * a.N0 * 8 < lim;
 }
 
-void launch_fft_pt(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
+bool launch_fft_pt(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   switch (a.n) {
-    case 36: launch_pt<6, 6>(a, ld_mode, st_mode, s); return;
-    case 48: launch_pt<6, 8>(a, ld_mode, st_mode, s); return;
-    case 54: launch_pt<6, 9>(a, ld_mode, st_mode, s); return;
-    case 64: launch_pt<8, 8>(a, ld_mode, st_mode, s); return;
-    case 72: launch_pt<8, 9>(a, ld_mode, st_mode, s); return;
-    case 81: launch_pt<9, 9>(a, ld_mode, st_mode, s); return;
-    case 96: launch_pt<8, 12>(a, ld_mode, st_mode, s); return;
-    case 108: launch_pt<9, 12>(a, ld_mode, st_mode, s); return;
-    case 128: launch_pt<8, 16>(a, ld_mode, st_mode, s); return;
-    case 144: launch_pt<12, 12>(a, ld_mode, st_mode, s); return;
+    case 36: return launch_pt<6, 6>(a, ld_mode, st_mode, s);
+    case 48: return launch_pt<6, 8>(a, ld_mode, st_mode, s);
+    case 54: return launch_pt<6, 9>(a, ld_mode, st_mode, s);
+    case 64: return launch_pt<8, 8>(a, ld_mode, st_mode, s);
+    case 72: return launch_pt<8, 9>(a, ld_mode, st_mode, s);
+    case 81: return launch_pt<9, 9>(a, ld_mode, st_mode, s);
+    case 96: return launch_pt<8, 12>(a, ld_mode, st_mode, s);
+    case 108: return launch_pt<9, 12>(a, ld_mode, st_mode, s);
+    case 128: return launch_pt<8, 16>(a, ld_mode, st_mode, s);
+    case 144: return launch_pt<12, 12>(a, ld_mode, st_mode, s);
     default: break;
   }
-  if (launch_fft_pt_b(a, ld_mode, st_mode, s) || launch_fft_pt_c(a, ld_mode, st_mode, s)) return;
-  (void)launch_fft_pt_d(a, ld_mode, st_mode, s);
+  return launch_fft_pt_b(a, ld_mode, st_mode, s) || launch_fft_pt_c(a, ld_mode, st_mode, s) ||
+         launch_fft_pt_d(a, ld_mode, st_mode, s);
 }
 
 }  // namespace cgs

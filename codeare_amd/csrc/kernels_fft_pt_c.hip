@@ -10,10 +10,10 @@ namespace cgs {
 
 bool launch_fft_pt_c(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   switch (a.n) {
-    case 324: launch_pt<18, 18>(a, ld_mode, st_mode, s); return true;
-    case 384: launch_pt<16, 24>(a, ld_mode, st_mode, s); return true;
-    case 432: launch_pt<18, 24>(a, ld_mode, st_mode, s); return true;
-    case 486: launch_pt<18, 27>(a, ld_mode, st_mode, s); return true;
+    case 324: return launch_pt<18, 18>(a, ld_mode, st_mode, s);
+    case 384: return launch_pt<16, 24>(a, ld_mode, st_mode, s);
+    case 432: return launch_pt<18, 24>(a, ld_mode, st_mode, s);
+    case 486: return launch_pt<18, 27>(a, ld_mode, st_mode, s);
     default: return false;
   }
 }

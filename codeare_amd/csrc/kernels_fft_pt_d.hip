@@ -10,9 +10,9 @@ namespace cgs {
 
 bool launch_fft_pt_d(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   switch (a.n) {
-    case 512: launch_pt<16, 32>(a, ld_mode, st_mode, s); return true;
-    case 576: launch_pt<24, 24>(a, ld_mode, st_mode, s); return true;
-    case 648: launch_pt<24, 27>(a, ld_mode, st_mode, s); return true;
+    case 512: return launch_pt<16, 32>(a, ld_mode, st_mode, s);
+    case 576: return launch_pt<24, 24>(a, ld_mode, st_mode, s);
+    case 648: return launch_pt<24, 27>(a, ld_mode, st_mode, s);
     default: return false;
   }
 }

@@ -308,7 +308,7 @@ bool fft_reg_supported(const FftArgs& a) {
   return (a.n == 256 || a.n == 384 || a.n == 512) && a.inner >= kRegLines && !a.That;
 }
 
-void launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
+bool launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   const int64_t nib = (a.inner + kRegLines - 1) / kRegLines;
   const dim3 grid((unsigned)(nib * a.outers));
 #define CGS_FFT8_CASE(L, S_)                                                                \
@@ -316,7 +316,7 @@ void launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
     if (a.n == 512) CGS_LAUNCH((k_fft_r8<8, L, S_>), grid, dim3(1024), 0, s, a);             \
     else if (a.n == 384) CGS_LAUNCH((k_fft_r8<6, L, S_>), grid, dim3(1024), 0, s, a);        \
     else CGS_LAUNCH((k_fft_r8<4, L, S_>), grid, dim3(1024), 0, s, a);                        \
-    return;                                                                                 \
+    return true;                                                                            \
   }
   CGS_FFT8_CASE(0, 0)
   CGS_FFT8_CASE(1, 0)
@@ -326,6 +326,7 @@ void launch_fft_reg(const FftArgs& a, int ld_mode, int st_mode, hipStream_t s) {
   CGS_FFT8_CASE(0, 1)
   CGS_FFT8_CASE(0, 2)
 #undef CGS_FFT8_CASE
+  return false;
 }
 
 }  // namespace cgs

@@ -330,7 +330,7 @@ static int fft_forward(Plan& p, int mode, const float2* src, const int* fl, cons
     fft_finish(a);
     const double b = bytes + (double)C * n0 * a.outer_per_frame * F * 8;
     Prof pr(p, CGS_K_FFT_FWD, b);
-    launch_fft(a, mode, 0, p.stream);
+    CHK(launch_fft(a, mode, 0, p.stream));
   }
   // pass 2, axis 1
   {
@@ -345,7 +345,7 @@ static int fft_forward(Plan& p, int mode, const float2* src, const int* fl, cons
     fft_finish(a);
     const double b = (double)C * n0 * (N1 + n1) * a.outer_per_frame * F * 8;
     Prof pr(p, CGS_K_FFT_FWD, b);
-    launch_fft(a, 0, 0, p.stream);
+    CHK(launch_fft(a, 0, 0, p.stream));
   }
   if (d == 3) {
     FftArgs a = fft_base(p, p.fa[2], -1);
@@ -359,7 +359,7 @@ static int fft_forward(Plan& p, int mode, const float2* src, const int* fl, cons
     fft_finish(a);
     const double b = (double)C * n0 * n1 * (N2 + n2) * F * 8;
     Prof pr(p, CGS_K_FFT_FWD, b);
-    launch_fft(a, 0, 0, p.stream);
+    CHK(launch_fft(a, 0, 0, p.stream));
   }
   return CGS_OK;
 }
@@ -376,7 +376,7 @@ static int fft_adjoint(Plan& p, float2* X, const int* fl) {
       a.inner = C * n0; a.outer_per_frame = 1; a.outers = F; a.fdone = fl;
       fft_finish(a);
       Prof pr(p, CGS_K_FFT_ADJ, (double)C * n0 * (n1 + N1) * F * 8);
-      launch_fft(a, 0, 0, p.stream);
+      CHK(launch_fft(a, 0, 0, p.stream));
     }
     {
       FftArgs a = fft_base(p, p.fa[0], +1);
@@ -385,7 +385,7 @@ static int fft_adjoint(Plan& p, float2* X, const int* fl) {
       a.inner = C; a.outer_per_frame = N1; a.outers = N1 * F; a.fdone = fl;
       fft_finish(a);
       Prof pr(p, CGS_K_FFT_ADJ, (double)C * (n0 + N0) * N1 * F * 8);
-      launch_fft(a, 0, 1, p.stream);
+      CHK(launch_fft(a, 0, 1, p.stream));
     }
   } else {
     {
@@ -395,7 +395,7 @@ static int fft_adjoint(Plan& p, float2* X, const int* fl) {
       a.inner = C * n0 * n1; a.outer_per_frame = 1; a.outers = F; a.fdone = fl;
       fft_finish(a);
       Prof pr(p, CGS_K_FFT_ADJ, (double)C * n0 * n1 * (n2 + N2) * F * 8);
-      launch_fft(a, 0, 0, p.stream);
+      CHK(launch_fft(a, 0, 0, p.stream));
     }
     {
       FftArgs a = fft_base(p, p.fa[1], +1);
@@ -404,7 +404,7 @@ static int fft_adjoint(Plan& p, float2* X, const int* fl) {
       a.inner = C * n0; a.outer_per_frame = N2; a.outers = N2 * F; a.fdone = fl;
       fft_finish(a);
       Prof pr(p, CGS_K_FFT_ADJ, (double)C * n0 * (n1 + N1) * N2 * F * 8);
-      launch_fft(a, 0, 0, p.stream);
+      CHK(launch_fft(a, 0, 0, p.stream));
     }
     {
       FftArgs a = fft_base(p, p.fa[0], +1);
@@ -413,7 +413,7 @@ static int fft_adjoint(Plan& p, float2* X, const int* fl) {
       a.inner = C; a.outer_per_frame = N1 * N2; a.outers = N1 * N2 * F; a.fdone = fl;
       fft_finish(a);
       Prof pr(p, CGS_K_FFT_ADJ, (double)C * (n0 + N0) * N1 * N2 * F * 8);
-      launch_fft(a, 0, 1, p.stream);
+      CHK(launch_fft(a, 0, 1, p.stream));
     }
   }
   return CGS_OK;
@@ -1583,8 +1583,9 @@ static int toeplitz_prepare(Plan& p) {
     hipError_t e = hipMemcpy(q.ybuf[0], wy.data(), sizeof(float2) * wy.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) { destroy_plan(q); set_error("copy of weights failed"); return CGS_ERR_HIP; }
   }
-  gridding(q, q.ybuf[0], false, nullptr);   // K(D) per frame -> q.Xc [f][(2N)^d]
-  fft_adjoint(q, q.Xc, nullptr);
+  rc = gridding(q, q.ybuf[0], false, nullptr);   // K(D) per frame -> q.Xc [f][(2N)^d]
+  if (rc == CGS_OK) rc = fft_adjoint(q, q.Xc, nullptr);
+  if (rc != CGS_OK) { destroy_plan(q); return rc; }
   // forward (2N)^d FFT of K, with K(D) at bin D mod 2N (the pad mapping with nin = n)
   const float2* src = q.Xc;
   float2* bufs[2] = {q.t1, q.grid};
@@ -1599,7 +1600,7 @@ static int toeplitz_prepare(Plan& p) {
     fa.outer_per_frame = upper;
     fa.outers = upper * F;
     fft_finish(fa);
-    launch_fft(fa, 0, 0, q.stream);
+    if ((rc = launch_fft(fa, 0, 0, q.stream)) != CGS_OK) { destroy_plan(q); return rc; }
     src = fa.out;
     lower *= N2[a];
   }
@@ -1767,7 +1768,7 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
   // block's coils into G partial images in p.Xc (store mode 2)
   auto pass = [&](int kind, const FftTab& tab, int sign, const float2* in, const float2* xin, float2* out, int nin,
                   int nout, int64_t inner, int64_t opf, int ld, const float* That, int64_t cells, double bytes,
-                  int st = 0) {
+                  int st = 0) -> int {
     FftArgs a = fft_base(p, tab, sign);
     a.in = in; a.x = xin; a.out = out;
     a.nin = nin; a.nout = nout;
@@ -1787,7 +1788,7 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
               (double)G * nout * (double)opf * 8;
     }
     Prof pr(p, kind, bytes * F);
-    launch_fft(a, ld, st, p.stream);
+    return launch_fft(a, ld, st, p.stream);
   };
   // 3D on the lean kernels too when every pass has one: the axis-0 pad and
   // crop treat the N1 N2 rows of a frame like the 2D kernels' N1 rows, the
@@ -1836,7 +1837,7 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
       Prof pr(p, CGS_K_TOEP_PAD, pad_bytes * F);
       launch_toep_pad(a, p.stream);
     } else {
-      pass(CGS_K_TOEP_PAD, p.ft[0], -1, nullptr, x, p.tt1, (int)N0, (int)M0, C, N1, 4, nullptr, 0, pad_bytes);
+      CHK(pass(CGS_K_TOEP_PAD, p.ft[0], -1, nullptr, x, p.tt1, (int)N0, (int)M0, C, N1, 4, nullptr, 0, pad_bytes));
     }
     const double conv_bytes = 2.0 * C * M0 * N1 * 8 + 4.0 * M0 * M1;
     if (lean3) {
@@ -1868,8 +1869,8 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
       Prof pr(p, CGS_K_TOEP_CONV, conv_bytes * F);
       launch_toep_conv(a, p.stream);
     } else {
-      pass(CGS_K_TOEP_CONV, p.ft[1], -1, p.tt1, nullptr, p.tt1, (int)N1, (int)N1, C * M0, 1, 0, p.That, M0,
-           conv_bytes);
+      CHK(pass(CGS_K_TOEP_CONV, p.ft[1], -1, p.tt1, nullptr, p.tt1, (int)N1, (int)N1, C * M0, 1, 0, p.That, M0,
+           conv_bytes));
     }
     if (lean_pc) {
       ToepArgs a = ta;
@@ -1882,13 +1883,13 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
       Prof pr(p, CGS_K_TOEP_CROP, bytes * F);
       launch_toep_crop(a, p.stream);
     } else {
-      pass(CGS_K_TOEP_CROP, p.ft[0], +1, p.tt1, nullptr, p.Xc, (int)M0, (int)N0, C, N1, 0, nullptr, 0, 0.0, 2);
+      CHK(pass(CGS_K_TOEP_CROP, p.ft[0], +1, p.tt1, nullptr, p.Xc, (int)M0, (int)N0, C, N1, 0, nullptr, 0, 0.0, 2));
     }
   } else {
-    pass(CGS_K_TOEP_PAD, p.ft[0], -1, nullptr, x, p.tt1, (int)N0, (int)M0, C, N1 * N2, 4, nullptr, 0,
-         ((double)(1 + C) * N0 * N1 * N2 + (double)C * M0 * N1 * N2) * 8);
-    pass(CGS_K_TOEP_PAD, p.ft[1], -1, p.tt1, nullptr, p.tt2, (int)N1, (int)M1, C * M0, N2, 0, nullptr, 0,
-         (double)C * M0 * (N1 + M1) * N2 * 8);
+    CHK(pass(CGS_K_TOEP_PAD, p.ft[0], -1, nullptr, x, p.tt1, (int)N0, (int)M0, C, N1 * N2, 4, nullptr, 0,
+         ((double)(1 + C) * N0 * N1 * N2 + (double)C * M0 * N1 * N2) * 8));
+    CHK(pass(CGS_K_TOEP_PAD, p.ft[1], -1, p.tt1, nullptr, p.tt2, (int)N1, (int)M1, C * M0, N2, 0, nullptr, 0,
+         (double)C * M0 * (N1 + M1) * N2 * 8));
     // the conv along axis 2 on the lean kernel: its lines run over the
     // (2 N0 x 2 N1) cells x C coils like the 2D kernel's over 2 N0 x C, so it
     // takes N0' = 2 N0 N1 (2 N0' cells) and N1' = N2
@@ -1900,12 +1901,12 @@ static int toeplitz_to_coils(Plan& p, const float2* x, const int* fl, const PUpd
       Prof pr(p, CGS_K_TOEP_CONV, conv3_bytes * F);
       launch_toep_conv(a, p.stream);
     } else {
-      pass(CGS_K_TOEP_CONV, p.ft[2], -1, p.tt2, nullptr, p.tt2, (int)N2, (int)N2, C * M0 * M1, 1, 0, p.That, M0 * M1,
-           conv3_bytes);
+      CHK(pass(CGS_K_TOEP_CONV, p.ft[2], -1, p.tt2, nullptr, p.tt2, (int)N2, (int)N2, C * M0 * M1, 1, 0, p.That, M0 * M1,
+           conv3_bytes));
     }
-    pass(CGS_K_TOEP_CROP, p.ft[1], +1, p.tt2, nullptr, p.tt1, (int)M1, (int)N1, C * M0, N2, 0, nullptr, 0,
-         (double)C * M0 * (M1 + N1) * N2 * 8);
-    pass(CGS_K_TOEP_CROP, p.ft[0], +1, p.tt1, nullptr, p.Xc, (int)M0, (int)N0, C, N1 * N2, 0, nullptr, 0, 0.0, 2);
+    CHK(pass(CGS_K_TOEP_CROP, p.ft[1], +1, p.tt2, nullptr, p.tt1, (int)M1, (int)N1, C * M0, N2, 0, nullptr, 0,
+         (double)C * M0 * (M1 + N1) * N2 * 8));
+    CHK(pass(CGS_K_TOEP_CROP, p.ft[0], +1, p.tt1, nullptr, p.Xc, (int)M0, (int)N0, C, N1 * N2, 0, nullptr, 0, 0.0, 2));
   }
   if (tail_out) *tail_out = (tail_parts == 2);
   return CGS_OK;
