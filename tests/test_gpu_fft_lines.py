@@ -41,15 +41,41 @@ def test_lines_match_oracle(cgs, ora, N, sigma, C):
     assert e3 <= (2e-5 if sigma == 2.0 else 2e-4)
 
 
+@pytest.mark.parametrize("N,C", [((24, 36, 32), 3), ((32, 24, 36), 10), ((36, 32, 24), 17), ((24, 32, 36), 1)])
+def test_volume_lines_match_oracle(cgs, ora, N, C):
+    """Volumes of three different sides (a row's place on the other two axes): errors as
+    in the plane."""
+    rng = np.random.default_rng(N[0] * 1000 + N[1] + C)
+    M = 500
+    k = rand_traj(rng, 3, M)
+    w = rng.uniform(0.2, 1.0, M).astype(np.float32)
+    S = rand_img(rng, N + (C,))
+    x, y = rand_img(rng, N), rand_img(rng, (M, C))
+    P = cgs.Plan(N, M, 1.5, 3, ncoils=C)
+    P.kspace(k)
+    P.weights(w)
+    P.sensitivities(S)
+    O = ora.NFFT(N, M, 1.5, 3)
+    O.kspace(k)
+    e1, e2 = rel(P.E(x), O.E(S, x)), rel(P.EH(y), O.EH_true(S, w, y))
+    e3 = rel(P.normal(x, lam=0.5, toeplitz=True), P.normal(x, lam=0.5))
+    print(f"{N} C={C}: E {e1:.2e}, E^H W {e2:.2e}, Toeplitz {e3:.2e}")
+    assert e1 <= 1e-5 and e2 <= 1e-5 and e3 <= 2e-4
+
+
 @pytest.mark.parametrize("N,C", [((32, 18), 3), ((48, 54), 1), ((36, 18), 10)])
 @pytest.mark.parametrize("toeplitz", [False, True])
 def test_rows_of_two_frames(cgs, N, C, toeplitz):
-    """Frames that stop at different iterations, with blocks that hold rows of two
-    frames: each frame equals its own solve of as many iterations."""
+    """Frames that stop at different iterations (weights of another scale against the
+    same lam), with blocks that hold rows of two frames, so that for some iterations a
+    block has a finished and a live one: each frame equals its own solve of as many
+    iterations."""
     rng = np.random.default_rng(N[0] + C)
     off = np.array([0, 300, 900, 1100], dtype=np.int64)
     k = rand_traj(rng, 2, int(off[-1]))
     w = rng.uniform(0.2, 1.0, int(off[-1])).astype(np.float32)
+    w[:off[1]] *= 1e-4
+    w[off[2]:] *= 1e-4
     S = rand_img(rng, N + (C,))
     x = rand_img(rng, N + (3,))
     P = cgs.Plan(N, int(off[-1]), 2.0, 3, ncoils=C, frame_offsets=off)
@@ -60,6 +86,7 @@ def test_rows_of_two_frames(cgs, N, C, toeplitz):
     xb, rb = P.solve(y, maxit=12, tol=0.2, lam=0.5, toeplitz=toeplitz)
     its = [int(i) for i in rb["iters"]]
     print(f"{N} C={C} toeplitz={toeplitz}: iterations {its}")
+    assert its[0] < its[1] and its[2] < its[1] < 12
     for f in range(3):
         Mf = int(off[f + 1] - off[f])
         P1 = cgs.Plan(N, Mf, 2.0, 3, ncoils=C)

@@ -26,7 +26,8 @@ def test_batch_equals_single_images(levels, H, W, B):
         assert np.array_equal(net.forward(x[i])[0], y[i])
 
 
-@pytest.mark.parametrize("levels,H,W,B", [(4, 128, 256, 8), (2, 32, 96, 16), (3, 64, 64, 2)])
+@pytest.mark.parametrize("levels,H,W,B", [(4, 128, 256, 8), (2, 32, 96, 16), (3, 64, 64, 2),
+                                           (5, 256, 256, 2), (6, 512, 512, 2)])   # 512 and 1024 channels
 def test_batch_gradient_is_mean_of_images(levels, H, W, B):
     """Sums of 1e5 FP32 products in two orders: 1e-5 of the gradient's norm per layer block."""
     from codeare_amd.warmstart import UNet
