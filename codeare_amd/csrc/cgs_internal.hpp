@@ -604,13 +604,13 @@ void launch_img_ext2coil(const Plan& p, const float2* ext, float2* X, int batch,
 void launch_img_coil2ext(const Plan& p, const float2* X, float2* ext, int batch, int frame,
                          hipStream_t s);
 // CGNR (reference E^H) kernels
-// step 1 / 2: also take the CGNR scalar step that reads this dot product (alpha / beta)
+// step: the CGNR scalar step that reads this dot product, taken with it: 3 the first stop
+// test (and the scalars' initial values), 0 the later ones, 1 alpha, 2 beta, -1 none
 void launch_cnr_dot(const Plan& p, const float2* v, int image, int slot, int step, double eps, const int* fl,
                     hipStream_t s);
 void launch_cnr_update(const Plan& p, float2* fhat, const float2* phat, bool first, const float2* rin, float2* r,
                        const float2* v, bool last, double eps, const int* fl, hipStream_t s);
 void launch_cnr_update_p(const Plan& p, float2* phat, const float2* z, const int* fl, hipStream_t s);
-void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 void launch_toep_layout(const float2* Khat, float* That, int64_t cells, int nl, int F, float scale,
                         hipStream_t s);
 void launch_fill_int(int* dst, int value, int n, hipStream_t s);

@@ -22,8 +22,11 @@
 // Measured against the kernels these lengths had before: 432- and 324-point
 // lines of 12 coils 22.4 -> 8.8 us a pass (LDS kernel, every stage through
 // LDS); the 96^3 x 8 coil Toeplitz iteration (192 points): convolution 340 ->
-// 135 us (3.6 TB/s), middle axis 84 -> 64, pad 89 -> 44, crop 98 -> 46; 192-point
-// lines of 16 coils in 3D 339 -> 235 us; 256-point lines of 8 coils 12 -> 7 us.
+// 129 us (3.7 TB/s), middle axis 84 -> 64, pad 89 -> 44, crop 98 -> 46; 192-point
+// lines of 16 coils in 3D 339 -> 235 us; 256-point lines of 8 coils 12 -> 7 us;
+// convolutions of 20 coils against 16 threads a line: 256 points 9.4 -> 9.0, 512
+// points 25.9 -> 21.2 us (16 frames 305 -> 270).  One and two coils on few rows go to
+// the LDS kernel (fft_few_rows, plan.hip).
 #pragma once
 
 #include "cgs_internal.hpp"

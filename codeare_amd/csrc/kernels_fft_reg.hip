@@ -15,7 +15,7 @@
 // against 21.3 us, last 15.0 against 23.1; 384 points 20.2 against 24.3 and 18.8
 // against 20.7.  At 256 points the two are level (19.5 against 19.1 us, 24
 // coils); below, k_fft_pt is faster (192 points, 16 coils in 3D: 235 against 339
-// us), and it takes every other length.
+// us), and it takes the other lengths from 36 to 648 points.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>

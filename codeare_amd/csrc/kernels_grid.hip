@@ -1216,14 +1216,15 @@ void launch_grid_mfma(const GridArgs& a, const int4* vrec, int nblocks, hipStrea
 // atomics.
 //
 // What bounds it: on the 128^3 koosh ball (5.12 M samples, 16 coils) the products left
-// are 2.8 ms of matrix work of 7.4 ms; the waves spend about half their time at the
-// batch's barrier and loads (the planes' visit counts of a batch differ), so the
-// register cap for three blocks a CU pays although it spills ten registers outside the
-// product loop (7.95 ms uncapped, two blocks).  Measured against one staged footprint
+// are 2.8 ms of matrix work of 7.0 ms (matrix cores 43 % busy, vector issue 41 %); the
+// waves spend about half their time at the batch's barrier and loads (the planes' visit
+// counts of a batch differ), so the register cap for three blocks a CU pays although it
+// spills ten registers outside the product loop (uncapped, two blocks: 7.95 against 7.4 ms
+// when it was chosen).  Measured against one staged footprint
 // placed per product, without double buffering (one work item of at most 4096 visits a
-// block in both): 10.2 -> 7.4 ms; 96^3 x 8 coils, 768 000 samples: 1.55 -> 0.60 ms.
-// Not kept: lane reads of the list instead of LDS reads (8.9 ms), items of 512-2048
-// visits (9.6-8.4 ms).
+// block in both): 10.2 -> 7.0 ms; 96^3 x 8 coils, 768 000 samples: 1.55 -> 0.62 ms.
+// Not kept, against 7.4 ms then: lane reads of the list instead of LDS reads (8.9 ms),
+// items of 512-2048 visits (9.6-8.4 ms).
 constexpr int kG3Batch = 64;
 template <int TAPS, int R, bool WIDE>
 __global__ void __launch_bounds__(512, 6) k_grid_mfma3(GridArgs a, const int4* __restrict__ vrec, int ngroups) {
@@ -1714,6 +1715,11 @@ __global__ void __launch_bounds__(NT, NT / 128) k_interp_lds3(SampArgs a, const 
 // by DPP steps (three or four, in place of five over 32 tap-row lanes).  Window
 // values and base cells come from global memory, one address per sample
 // broadcast to its lanes, so only the region sits in LDS.
+// What bounds it: vector issue.  On the 128^3 koosh ball with 16 coils its 1.17 M waves
+// issue 2406 vector instructions each, 4.6 ms at one a CU and cycle, of the 4.7-5.0 ms it
+// takes (the tap FMAs alone are 2.1 ms); the LDS is 88 % busy, a third of that bank
+// conflicts.  Before an item's coil pairs ran one after the other on one XCD: 6.5 ms, 34
+// instead of 4.3 GB fetched.
 template <int TAPS, int NT, int TT, int SPLIT>
 __global__ void __launch_bounds__(NT, NT / 128) k_interp_cs3(SampArgs a, const int4* items, int nitems, int ngroups,
                                                              int T_, int nt0, int nt1, int ppad) {

@@ -1145,10 +1145,6 @@ void launch_toep_layout(const float2* Khat, float* That, int64_t cells, int nl, 
   hipLaunchKernelGGL(k_toep_layout, dim3(2048), dim3(256), 0, s, Khat, That, cells, nl, F, scale);
 }
 
-void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
-  (void)hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, s);
-}
-
 __global__ void k_fill_int(int* dst, int v, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = v;

@@ -5,9 +5,10 @@
 // Tensors are NHWC: activation[((b*H + y)*W + x)*C + c], BF16 storage.  The
 // network input and output are complex64 images, i.e. NHWC with C = 2
 // (re, im).  Conv weights are kept as FP32 masters [tap][co][ci] (tap = 3*ky+kx)
-// with a BF16 copy in that layout for the forward pass and a flipped, transposed
-// BF16 copy [8-tap][ci][co] for the input-gradient pass, which is then the same
-// convolution kernel.  Every reduction (weight and bias gradients, loss) runs in
+// with BF16 copies in the order the matrix instructions take them (k_wprep): one of
+// the weights for the forward pass, one of the flipped, transposed weights
+// W'[8-tap][ci][co] for the input-gradient pass, which is then the same convolution
+// kernel (none for the first layer: nothing takes its input's gradient).  Every reduction (weight and bias gradients, loss) runs in
 // a fixed order, so a training step is deterministic.
 //
 // There is no counterpart in codeare: the network supplies x0 for the CG solve
@@ -914,7 +915,7 @@ int prep_weights(cgs_unet_s& n) {
     const int Cin = c.ca + c.cb;
     const size_t nw = (size_t)9 * c.cout * Cin;
     hipLaunchKernelGGL(k_wprep, dim3(grid_for(nw)), dim3(256), 0, n.stream, (const float*)(n.params + c.w_off), c.wf,
-                       Cin % 32 ? nullptr : c.wb, c.cout, Cin);
+                       c.wb, c.cout, Cin);
     UCHK(hipGetLastError());
   }
   return CGS_OK;
@@ -1066,8 +1067,9 @@ int upload(cgs_unet_s& n, const void* x, int batch, int device_io, const float2*
 
 }  // namespace
 
-// n normal values of deviation sd.  Aligned and on its own: where the linker puts
-// this loop (two million values) decides between 77 and 133 ms of a network's creation
+// n normal values of deviation sd.  On its own and aligned because its time (two
+// million values, most of a network's creation) came out at 77 or at 133 ms from one
+// link of the same objects to the next; what decides is not known
 static __attribute__((noinline, aligned(64))) void normal_fill(float* w, size_t n, float sd, std::mt19937_64& rng) {
   std::normal_distribution<float> nd(0.f, sd);
   for (size_t i = 0; i < n; ++i) w[i] = nd(rng);
@@ -1132,7 +1134,8 @@ int cgs_unet_create(cgs_unet* out, int H, int W, int levels, int base_channels, 
     return fail(rc);
   for (auto& c : n->convs) {
     const size_t nw = (size_t)9 * c.cout * (c.ca + c.cb);
-    if ((rc = dmalloc(&c.wf, nw)) || (rc = dmalloc(&c.wb, nw))) return fail(rc);
+    const bool first = (c.ca + c.cb) % 32 != 0;   // its input's gradient is not formed
+    if ((rc = dmalloc(&c.wf, nw)) || (!first && (rc = dmalloc(&c.wb, nw)))) return fail(rc);
   }
   const size_t B = max_batch;
   n->act_a.assign(levels, nullptr);
