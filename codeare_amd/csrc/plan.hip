@@ -1691,12 +1691,16 @@ static bool toep_pad_row_enabled(int C) {   // CGS_TOEP_PAD_ROW=0: one block per
   return on && toep_row_shape(C);
 }
 
-// frames per run of the three passes below: their grid, written by one pass and
-// read by the next, then stays in the 256 MB last-level cache instead of going
-// to memory and back.  192^2 x 16 coils x 64 frames (9.4 MB of grid a frame),
-// CG(20): all frames at once 15.64 ms, 16 frames 15.14, 12 frames 14.75, 8 frames
-// 15.61 (the launches then fill the chip for too short a time).
-constexpr double kToepRunBytes = 128.0 * 1048576.0;
+// The three passes below go over a series in runs of frames where its grid, written by
+// one pass and read by the next, would not stay in the 256 MB last-level cache: as many
+// runs as whole times this size fit, so the grids of 1, 2, 3 .. runs reach 224, 168, 149 ..
+// MiB before there is one more.  Up to 224 MiB one run is best, because every launch's
+// ramp and drain count: 16 coils, CG(20), all frames at once against two runs, 192^2 x 15
+// frames (135 MiB) 3.45 / 3.83 ms, 256^2 x 12 (192 MiB) 4.34 / 4.75, 192^2 x 24 (216 MiB)
+// level, 128^2 x 56 (224 MiB) 5.98 / 5.75, 256^2 x 16 (256 MiB) 6.41 / 5.97.  Beyond, fewer and
+// longer runs: 192^2 x 32 (288 MiB) 7.90 at once, 6.95 in two, 7.55 in three; x 64 (576 MiB)
+// 15.5 at once, 14.5 in five (117 MiB each), 15.0 in six.
+constexpr double kToepRunBytes = 112.0 * 1048576.0;
 
 // The three lean passes of the 2D operator (kernels_toep.hip), run by run of
 // frames; *G_out partial images per frame in p.Xc.
@@ -1705,8 +1709,8 @@ static void toeplitz_lean_2d(Plan& p, const float2* x, const int* fl, const PUpd
   const int C = p.C, F = p.F;
   const int64_t N0 = p.N[0], N1 = p.N[1], M0 = 2 * N0, M1 = 2 * N1;
   const double gbytes = (double)C * M0 * N1 * 8;   // a frame's grid
-  const int most = (int)std::max(1.0, std::min((double)F, kToepRunBytes / gbytes));
-  const int runs = (F + most - 1) / most, per = (F + runs - 1) / runs;
+  const int runs = (int)std::max(1.0, std::min((double)F, std::floor(F * gbytes / kToepRunBytes)));
+  const int per = (F + runs - 1) / runs;
   const bool row = toep_row_enabled(C);
   const int G = row ? 1 : C / 16;
   *G_out = G;

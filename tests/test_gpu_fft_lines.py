@@ -100,9 +100,9 @@ def test_rows_of_two_frames(cgs, N, C, toeplitz):
 
 @pytest.mark.parametrize("graph", [0, 3])
 def test_toeplitz_runs_of_frames(cgs, graph):
-    """15 frames of 192^2 x 16 coils: the Toeplitz passes go over them in two runs
-    (8 and 7 frames); frames at the ends of both runs equal their own solves."""
-    N, C, F, Mf = (192, 192), 16, 15, 250
+    """25 frames of 192^2 x 16 coils: the Toeplitz passes go over them in two runs
+    (13 and 12 frames); frames at the ends of both runs equal their own solves."""
+    N, C, F, Mf = (192, 192), 16, 25, 250
     rng = np.random.default_rng(192)
     off = np.arange(F + 1, dtype=np.int64) * Mf
     k = rand_traj(rng, 2, F * Mf)
@@ -116,7 +116,7 @@ def test_toeplitz_runs_of_frames(cgs, graph):
     xb, rb = P.solve(y, maxit=6, tol=0.0, lam=0.5, toeplitz=True, graph_iters=graph)
     P1 = cgs.Plan(N, Mf, 2.0, 3, ncoils=C)
     P1.sensitivities(S)
-    for f in (0, 7, 8, 14):
+    for f in (0, 12, 13, 24):
         P1.kspace(k[:, off[f]:off[f + 1]])
         P1.weights(w[off[f]:off[f + 1]])
         yf = y[C * off[f]:C * off[f + 1]].reshape((Mf, C), order="F")
